@@ -40,6 +40,31 @@ def test_encode_bit_exact(rng):
     assert np.array_equal(_bits(gf), fac)
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 130])
+def test_encode_tile_edges_and_nonfinite_rows(rng, n):
+    """A partial tile of 64 rows, and rows with infinities and NaNs: codes as
+    the oracle's (y >= 0 is false for a NaN), factors equal or both NaN."""
+    from zoomkv_revision_amd.rabitq import rabitq_encode
+    s_np, s_t = _signs(11)
+    x = (rng.standard_normal((n, 128)) * 3).astype(np.float32)
+    x[0, 17] = np.inf                                        # one infinity: no NaN in y
+    if n > 60:
+        x[1, 3], x[1, 90] = -np.inf, np.inf                  # two: some y are NaN
+        x[2, [5, 6, 7, 101]] = np.inf
+        x[3, 64] = np.nan
+        x[4, 64], x[4, 9] = np.nan, -np.inf
+        x[n - 1] = -0.0
+    keys = f16_bits(x)
+    with np.errstate(invalid="ignore"):
+        codes, fac = orq.encode(keys, s_np)
+    gc, gf = rabitq_encode(_f16(keys), s_t)
+    assert np.array_equal(from_torch(gc), codes)
+    got, want = _bits(gf), fac
+    nan = np.isnan(want.view(np.float16))
+    assert np.array_equal(np.isnan(got.view(np.float16)), nan)
+    assert np.array_equal(got[~nan], want[~nan])
+
+
 def test_encode_strided_rows(rng):
     from zoomkv_revision_amd.rabitq import rabitq_encode
     s_np, s_t = _signs(3)

@@ -137,17 +137,6 @@ constexpr int kRecordWords = kStageBytes / 4;
 // first half of its group takes the second half's places, which the tile
 // compute treats alike), plus page B's K scale/zero slots at [5120, 5632).
 constexpr int kPairStageBytes = 5632;
-// cache policy of the tile loads: nt (streamed once, not kept in the caches)
-constexpr int kCachePolicyNT = 2;
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-// 64 lanes x 16 B from per-lane global addresses straight into LDS at
-// dst + 16*lane (global_load_lds_dwordx4): the prefetch ring costs no VGPRs.
-__device__ __forceinline__ void dma16(const void* src, void* dst) {
-  __builtin_amdgcn_global_load_lds(src, (lds_void_t*)(dst), 16, 0, kCachePolicyNT);
-}
-
 // LDS byte address of a pointer into __shared__ memory.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const lds_void_t*)(p)));
@@ -162,14 +151,6 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // M0; lane i lands at dst + 16 i).
 __device__ __forceinline__ void dma16_untracked(const void* src, void* dst) {
   asm volatile("global_load_lds_dwordx4 %0, off nt" : : "v"(src), "{m0}"(lds_addr(dst)) : "memory");
-}
-
-// s_waitcnt vmcnt(n) (gfx9 encoding: vmcnt[3:0] bits 3:0, vmcnt[5:4] bits
-// 15:14; expcnt / lgkmcnt left at "no wait").  The compiler does not track the
-// LDS side of global_load_lds, so the ring's waits are explicit.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N & 0x30) << 10) | 0x0F70);
 }
 
 __device__ __forceinline__ void wait_tiles_in_flight(int later) {

@@ -36,32 +36,77 @@ __device__ __forceinline__ float f16_to_f32(uint16_t h) {
 }
 
 // ----------------------------------------------------------------------------
-// Encode: one thread per vector (its sums are sequential in dimension order).
+// Encode: one lane per vector (its three sums are sequential in dimension
+// order), one wave per workgroup and tile of 64 vectors.  Bound: HBM (276 B
+// per vector), with the butterfly's and the sums' ~1650 VALU instructions per
+// tile close behind.  The tile comes in through LDS: a lane that loads its
+// own row from memory touches 64 lines per instruction, which the L1 cannot
+// hold until their other chunks are asked for.  Sixteen-KiB workgroups of one
+// wave need no barrier and run 10 to a CU, so that some load while others
+// compute.  1,048,576 vectors: 63 us (4.6 TB/s; a plain device copy moves 5.1
+// TB/s here) against 123 us with per-lane loads from memory.
 // ----------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void rabitq_encode_kernel(
+// The code of a row that holds infinities or NaNs (finite fp16 rows cannot
+// overflow the butterfly): bit j is y_j >= 0.  A NaN makes every y a NaN;
+// otherwise y_j is +inf where every infinite dimension d enters it with a
+// positive sign, (-1)^popc(j & d) sign_d sgn(x_d) > 0, and -inf or NaN elsewhere.
+__device__ __forceinline__ u32x4_t nonfinite_code(const uint8_t* tile, int row,
+                                                  const float* __restrict__ signs) {
+  u32x4_t code = {~0u, ~0u, ~0u, ~0u};
+#pragma unroll 1
+  for (int d = 0; d < kD; ++d) {
+    const uint32_t h = *reinterpret_cast<const uint16_t*>(tile + row_tile_offset(row, d >> 3) + 2 * (d & 7));
+    if ((h & 0x7C00u) != 0x7C00u) continue;
+    if (h & 0x03FFu) {
+      code = u32x4_t{0u, 0u, 0u, 0u};
+      break;
+    }
+    uint32_t low = 0u;  // bit b: the parity of popc(b & d) over b < 32
+    if (d & 1) low ^= 0xAAAAAAAAu;
+    if (d & 2) low ^= 0xCCCCCCCCu;
+    if (d & 4) low ^= 0xF0F0F0F0u;
+    if (d & 8) low ^= 0xFF00FF00u;
+    if (d & 16) low ^= 0xFFFF0000u;
+    if ((h >> 15) != (signs[d] < 0.0f ? 1u : 0u)) low = ~low;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) code[w] &= (__popc(w & (d >> 5)) & 1) ? low : ~low;
+  }
+  return code;
+}
+
+__global__ __launch_bounds__(64, 3) void rabitq_encode_kernel(
     const uint16_t* __restrict__ x, int64_t row_stride, int64_t n, const float* __restrict__ signs,
     uint8_t* __restrict__ codes, uint16_t* __restrict__ factors) {
-  __shared__ float s_sign[kD];
-  if (threadIdx.x < kD) s_sign[threadIdx.x] = signs[threadIdx.x];
-  __syncthreads();
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const u32x4_t* row = reinterpret_cast<const u32x4_t*>(x + i * row_stride);
+  __shared__ __attribute__((aligned(16))) uint8_t tile[kRowTileBytes];
+  const int lane = threadIdx.x;
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * 64;
+  load_row_tile(tile, x + i0 * row_stride, row_stride, static_cast<int>(min(n - i0, static_cast<int64_t>(64))));
   float y[kD];
   float nsq = 0.0f;
 #pragma unroll
   for (int c = 0; c < kD / 8; ++c) {
-    const u32x4_t w = row[c];
+    const u32x4_t w = row_tile_chunk(tile, lane, c);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint16_t h = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
-      const float v = f16_to_f32(h);
-      nsq = nsq + v * v;
-      y[8 * c + e] = v * s_sign[8 * c + e];
+    for (int e = 0; e < 4; ++e) {
+      const half2_t h = u32_as_half2(w[e]);
+      const float a = static_cast<float>(h[0]), b = static_cast<float>(h[1]);
+      // products of two fp16 values, and of an fp16 value and +-1, are exact in
+      // fp32: the multiply-adds round as a multiply and an add do
+      nsq = __builtin_fmaf(a, a, nsq);
+      nsq = __builtin_fmaf(b, b, nsq);
+      // the signs and the butterfly's first stage.  (+ 0 leaves no -0 here, so
+      // none arises in the later stages: the sign bit below is y < 0.)
+      const int d = 8 * c + 2 * e;
+      const float t = __builtin_fmaf(a, signs[d], 0.0f);
+      y[d] = __builtin_fmaf(b, signs[d + 1], t);
+      y[d + 1] = __builtin_fmaf(-b, signs[d + 1], t);
     }
+    // (each sum is pinned where it is formed: sunk to its use below, it would
+    // keep all the row's words, or all of y, in registers and spill)
+    asm volatile("" : "+v"(nsq));
   }
 #pragma unroll
-  for (int h = 1; h < kD; h <<= 1) {
+  for (int h = 2; h < kD; h <<= 1) {
 #pragma unroll
     for (int b0 = 0; b0 < kD; b0 += 2 * h) {
 #pragma unroll
@@ -73,13 +118,23 @@ __global__ __launch_bounds__(256) void rabitq_encode_kernel(
     }
   }
   float ysq = 0.0f, yabs = 0.0f;
-  u32x4_t code = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int d = 0; d < kD; ++d) {
     ysq = ysq + y[d] * y[d];
     yabs = yabs + fabsf(y[d]);
-    code[d >> 5] |= static_cast<uint32_t>(y[d] >= 0.0f) << (d & 31);
   }
+  asm volatile("" : "+v"(ysq), "+v"(yabs));
+  u32x4_t code;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    uint32_t neg = 0u;  // shifted left once per dimension, highest first
+#pragma unroll
+    for (int d = 31; d >= 0; --d) neg = __builtin_amdgcn_alignbit(neg, __float_as_uint(y[32 * w + d]), 31);
+    code[w] = ~neg;
+  }
+  if (!(yabs < INFINITY)) code = nonfinite_code(tile, lane, signs);
+  if (i0 + lane >= n) return;
+  const int64_t i = i0 + lane;
   const float norm = sqrtf(nsq);
   const float corr = yabs > 0.0f ? (sqrtf(ysq) * kSqrt128) / yabs : 0.0f;
   *reinterpret_cast<u32x4_t*>(codes + i * 16) = code;
@@ -1613,8 +1668,8 @@ SearchLayout search_layout(int pools, int queries, int64_t n, int topk) {
 int launch_encode(const uint16_t* x, int64_t row_stride, int64_t n, const float* signs, uint8_t* codes,
                   uint16_t* factors, hipStream_t stream) {
   if (n == 0) return ZKV_OK;
-  const unsigned blocks = static_cast<unsigned>((n + 255) / 256);
-  rabitq_encode_kernel<<<blocks, 256, 0, stream>>>(x, row_stride, n, signs, codes, factors);
+  const unsigned blocks = static_cast<unsigned>((n + 63) / 64);
+  rabitq_encode_kernel<<<blocks, 64, 0, stream>>>(x, row_stride, n, signs, codes, factors);
   return check_launch("rabitq_encode_kernel");
 }
 

@@ -155,6 +155,57 @@ __device__ __forceinline__ void nibbles_to_half_pairs(uint32_t w, half2_t out[4]
 }
 
 // ---------------------------------------------------------------------------
+// Global memory straight into LDS
+// ---------------------------------------------------------------------------
+// cache policy of streamed loads: nt (read once, not kept in the caches)
+constexpr int kCachePolicyNT = 2;
+
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// 64 lanes x 16 B from per-lane global addresses straight into LDS at
+// dst + 16*lane (global_load_lds_dwordx4): the data in flight costs no VGPRs.
+__device__ __forceinline__ void dma16(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds(src, (lds_void_t*)(dst), 16, 0, kCachePolicyNT);
+}
+
+// s_waitcnt vmcnt(n) (gfx9 encoding: vmcnt[3:0] bits 3:0, vmcnt[5:4] bits
+// 15:14; expcnt / lgkmcnt left at "no wait").  The compiler does not track the
+// LDS side of global_load_lds, so the waits for it are explicit.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N & 0x30) << 10) | 0x0F70);
+}
+
+// A wave's tile of 64 rows of 256 bytes (128 16-bit values) for kernels that
+// give each lane one whole row.  The rows come in as 16 coalesced DMAs of 4
+// rows; 16-byte chunk c of row r lands in slot c ^ (r & 15) of its row, so
+// that the 16 lanes of a read phase, each reading chunk c of its own row, hit
+// 16 different slots (all 64 banks once).  Row r < rows is at base + r *
+// stride (uint16 units, 16-byte aligned); rows past the end repeat the last.
+// Returns when the tile is there; only the wave itself reads it.
+constexpr int kRowTileBytes = 64 * 256;
+__device__ __forceinline__ void load_row_tile(uint8_t* tile, const uint16_t* base, int64_t stride, int rows) {
+  const int lane = threadIdx.x & 63, r0 = lane >> 4;
+  // chunk lane % 16 of row 4 i + r0 comes from chunk (lane ^ row) % 16
+  if (rows >= 64) {
+    const uint16_t* p = base + r0 * stride;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      dma16(p + 4 * i * stride + 8 * ((lane ^ (4 * i + r0)) & 15), tile + 1024 * i);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      dma16(base + min(4 * i + r0, rows - 1) * stride + 8 * ((lane ^ (4 * i + r0)) & 15), tile + 1024 * i);
+  }
+  wait_vmcnt<0>();
+  asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ int row_tile_offset(int r, int c) { return 256 * r + 16 * (c ^ (r & 15)); }
+__device__ __forceinline__ u32x4_t row_tile_chunk(const uint8_t* tile, int r, int c) {
+  return *reinterpret_cast<const u32x4_t*>(tile + row_tile_offset(r, c));
+}
+
+// ---------------------------------------------------------------------------
 // In-launch arrival counts: the workgroups of one unit of work (the context
 // splits of one (b, kv) attention) count themselves in on an 8-byte slot
 // (epoch << 8) | count; the one that completes the count does the unit's
