@@ -87,3 +87,29 @@ def test_zeros_keep_their_sign_only_with_the_select():
     z = np.array([0.0, -0.0], dtype=np.float32)
     got = div_recip(z, np.full(2, 15.0, dtype=np.float32))
     assert np.array_equal(got.view(np.uint32), np.zeros(2, dtype=np.uint32))
+
+
+def _bf16_rne(x: np.ndarray) -> np.ndarray:
+    u = x.astype(np.float32).view(np.uint32).astype(np.uint64)
+    return ((u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint32)
+
+
+def test_bf16_quotient_by_reciprocal_product():
+    """bf16(x / d) == bf16(x * (1 / d)) for bf16 x and d (rabitq4.hip's encode):
+    every pair of significands, with quotients from overflow down through
+    bf16's subnormal range, and with the reciprocal off by one unit in the
+    last place (the hardware's) where the quotient is normal."""
+    sig = 1.0 + np.arange(128, dtype=np.float64) / 128.0
+    xs, ds = np.meshgrid(sig, sig, indexing="ij")
+    for ex, ed in [(0, 0), (127, 0), (127, -1), (127, -26), (-60, 67), (100, 127), (-126, 0)] + \
+            [(-60, e) for e in range(63, 80)]:
+        x = np.ldexp(xs, ex).astype(np.float32)
+        d = np.ldexp(ds, ed).astype(np.float32)
+        with np.errstate(over="ignore"):
+            ref = _bf16_rne(x / d)
+            r = (np.float32(1.0) / d).astype(np.float32)
+            assert np.array_equal(_bf16_rne((x * r).astype(np.float32)), ref), (ex, ed)
+            if -100 < ex - ed < 120:
+                for to in (np.float32(0), np.float32(np.inf)):
+                    near = np.nextafter(r, to)
+                    assert np.array_equal(_bf16_rne((x * near).astype(np.float32)), ref), (ex, ed, to)

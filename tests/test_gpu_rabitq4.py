@@ -96,6 +96,61 @@ def test_encode_matches_oracle_strided_append(rng, bs, kv, n, t0, cap):
     assert (p_np[..., t0 + n:, :] == 0xCD).all()
 
 
+def _edge_keys(g, n):
+    """bf16 rows for the encode's special cases between ordinary ones."""
+    x = torch.randn(n, 128, generator=g, device="cuda") * torch.rand(n, 1, generator=g, device="cuda") * 30
+    x[1] = 0.0
+    x[2] = -0.0
+    x[3, 64:72] = 0.0
+    x[4] *= 1e-23                      # squares below fp32's normal range
+    x[5] *= 1e-38                      # subnormal values
+    x[6] *= 1e18                       # the sum of squares overflows
+    x[7], x[8], x[9] = 3e38, 1e-8, -1e-8
+    x[10, 5] = float("nan")
+    x[11, 100] = float("inf")
+    x[12, 3], x[12, 70] = float("-inf"), float("inf")
+    x[13] *= 1e-12                     # two equal entries cancel in half of y, leaving small blocks
+    x[13, 0] = x[13, 64] = 5.0
+    x[14] *= 1e-25
+    x[14, 0] = x[14, 64] = 5.0
+    x[15] = 1.0
+    return x.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("bs,kv,n,t0,thresholds", [
+    (1, 1, 41024, 0, None),                      # whole tiles
+    (1, 5, 8261, 3, None),                       # a last tile of 5 keys, odd first token
+    (2, 3, 7039, 1, "small"),                    # a threshold below the table: the general path in the tiles' launch
+    (1, 8, 5184, 0, "unsorted"),                 # counts of unsorted, negative and equal levels
+])
+def test_encode_tiles_match_short_calls(bs, kv, n, t0, thresholds):
+    """Calls of 40960 keys and more (a lane per key) write the bits of calls of
+    a few keys (16 lanes per key, checked against the oracle above), special
+    rows included; NaN weights are NaN in both."""
+    zk = _zk()
+    g = torch.Generator(device="cuda").manual_seed(5)
+    keys = torch.stack([_edge_keys(g, n) for _ in range(bs * kv)]).view(bs, kv, n, 128)
+    signs = (torch.randint(0, 2, (128,), generator=g, device="cuda") * 2 - 1).to(torch.bfloat16)
+    thr, ctr = _levels(zk)
+    if thresholds == "small":
+        thr = thr * 0 + torch.tensor([0.0, 1e-3, 0.02, 0.1, 0.3, 0.5, 0.9], device="cuda").to(torch.bfloat16)
+    elif thresholds == "unsorted":
+        thr = torch.tensor([0.5, -0.25, 0.125, 0.125, 2.0, 0.01, 0.75], device="cuda").to(torch.bfloat16)
+    mk = lambda: (torch.full((bs, kv, 16, t0 + n + 2), 0xAB, dtype=torch.uint8, device="cuda"),
+                  torch.full((bs, kv, 16, t0 + n + 2), 7.0, dtype=torch.bfloat16, device="cuda"),
+                  torch.full((bs, kv, 16, t0 + n + 2, 4), 0xCD, dtype=torch.uint8, device="cuda"))
+    got, want = mk(), mk()
+    assert bs * kv * n >= 40960
+    zk.encode_into(keys, signs, thr, ctr, *got, t0)
+    for i in range(0, n, 2000):
+        zk.encode_into(keys[:, :, i:i + 2000], signs, thr, ctr, *want, t0 + i)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2])
+    nan = torch.isnan(want[1])
+    assert torch.equal(torch.isnan(got[1]), nan)
+    assert torch.equal(got[1].view(torch.int16)[~nan], want[1].view(torch.int16)[~nan])
+
+
 def test_query_blocks_match_oracle(rng):
     zk = _zk()
     sg = np.where(rng.integers(0, 2, 128) == 1, 1.0, -1.0).astype(np.float32)

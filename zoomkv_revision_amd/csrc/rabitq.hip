@@ -55,7 +55,7 @@ __device__ __forceinline__ u32x4_t nonfinite_code(const uint8_t* tile, int row,
   u32x4_t code = {~0u, ~0u, ~0u, ~0u};
 #pragma unroll 1
   for (int d = 0; d < kD; ++d) {
-    const uint32_t h = *reinterpret_cast<const uint16_t*>(tile + row_tile_offset(row, d >> 3) + 2 * (d & 7));
+    const uint32_t h = *reinterpret_cast<const uint16_t*>(tile + row_tile_offset<16>(row, d >> 3) + 2 * (d & 7));
     if ((h & 0x7C00u) != 0x7C00u) continue;
     if (h & 0x03FFu) {
       code = u32x4_t{0u, 0u, 0u, 0u};
@@ -77,15 +77,15 @@ __device__ __forceinline__ u32x4_t nonfinite_code(const uint8_t* tile, int row,
 __global__ __launch_bounds__(64, 3) void rabitq_encode_kernel(
     const uint16_t* __restrict__ x, int64_t row_stride, int64_t n, const float* __restrict__ signs,
     uint8_t* __restrict__ codes, uint16_t* __restrict__ factors) {
-  __shared__ __attribute__((aligned(16))) uint8_t tile[kRowTileBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t tile[64 * 256];
   const int lane = threadIdx.x;
   const int64_t i0 = static_cast<int64_t>(blockIdx.x) * 64;
-  load_row_tile(tile, x + i0 * row_stride, row_stride, static_cast<int>(min(n - i0, static_cast<int64_t>(64))));
+  load_row_tile<16>(tile, x + i0 * row_stride, row_stride, static_cast<int>(min(n - i0, static_cast<int64_t>(64))));
   float y[kD];
   float nsq = 0.0f;
 #pragma unroll
   for (int c = 0; c < kD / 8; ++c) {
-    const u32x4_t w = row_tile_chunk(tile, lane, c);
+    const u32x4_t w = row_tile_chunk<16>(tile, lane, c);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const half2_t h = u32_as_half2(w[e]);

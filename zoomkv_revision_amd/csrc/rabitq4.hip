@@ -48,10 +48,10 @@ __device__ __forceinline__ float srht_unit_block(const float x[8], const float s
 #pragma unroll
   for (int d = 8; d >= 1; d >>= 1) s = s + shfl_xor(s, d);
   const float nrm = bf16r(__builtin_sqrtf(s));
-  const float den = fmaxf(nrm, kBf16OneEm8);
+  const float rden = 1.0f / fmaxf(nrm, kBf16OneEm8);  // bf16(x rden) = bf16(x / den), as below
   float v[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = bf16r(x[j] / den) * sg[j];
+  for (int j = 0; j < 8; ++j) v[j] = bf16r(x[j] * rden) * sg[j];
 #pragma unroll
   for (int h = 1; h < 8; h <<= 1)
 #pragma unroll
@@ -93,6 +93,9 @@ struct EncodeParams {
   const uint16_t* ctr;
 };
 
+// Sums of squares below this may hold products below fp32's normal range.
+constexpr float kTinySum = 0x1p-100f;
+
 __device__ __forceinline__ void load_row8(const uint16_t* p, float x[8]) {
   const u32x4_t r = *reinterpret_cast<const u32x4_t*>(p);
 #pragma unroll
@@ -102,11 +105,11 @@ __device__ __forceinline__ void load_row8(const uint16_t* p, float x[8]) {
   }
 }
 
-__global__ __launch_bounds__(256) void rabitq4_encode_kernel(const EncodeParams p) {
-  const int64_t row = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) >> 4;
-  const int blk = threadIdx.x & 15;
-  // rows past the end repeat the last row (every lane of a 16-lane group
-  // takes part in the shuffles) and store nothing
+// One key on 16 lanes (lane blk holds block blk): for launches of few keys,
+// where a lane per key would leave most of the chip idle, and for thresholds
+// the lookup table below cannot hold.  Rows past the end repeat the last row
+// (every lane of a 16-lane group takes part in the shuffles) and store nothing.
+__device__ __forceinline__ void encode_key16(const EncodeParams& p, int64_t row, int blk) {
   const int64_t r = row < p.rows ? row : p.rows - 1;
   const int64_t bh = r / p.n;
   const int t = static_cast<int>(r - bh * p.n);
@@ -126,13 +129,13 @@ __global__ __launch_bounds__(256) void rabitq4_encode_kernel(const EncodeParams 
 #pragma unroll
   for (int j = 0; j < 8; ++j) s = s + y[j] * y[j];
   const float rad = bf16r(__builtin_sqrtf(s));
-  const float den = fmaxf(rad, kBf16OneEm8);
+  const float rden = 1.0f / fmaxf(rad, kBf16OneEm8);
   uint32_t code = 0, packed = 0;
   float alpha = 0.0f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const uint32_t sb = y[j] >= 0.0f ? 1u : 0u;
-    const float au = fabsf(bf16r(y[j] / den));
+    const float au = fabsf(bf16r(y[j] * rden));
     uint32_t tq = 0;
 #pragma unroll
     for (int i = 0; i < 7; ++i) tq += au > thr[i] ? 1u : 0u;
@@ -150,6 +153,221 @@ __global__ __launch_bounds__(256) void rabitq4_encode_kernel(const EncodeParams 
     p.code[b * p.c_sb + h * p.c_sh + blk * p.c_sB + tt] = static_cast<uint8_t>(code);
     p.packed[b * p.p_sb + h * p.p_sh + blk * p.p_sB + tt] = packed;
     p.weight[b * p.w_sb + h * p.w_sh + blk * p.w_sB + tt] = f32_to_bf16_bits(w);
+  }
+}
+
+__global__ __launch_bounds__(256) void rabitq4_encode_small_kernel(const EncodeParams p) {
+  encode_key16(p, (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) >> 4, threadIdx.x & 15);
+}
+
+// The bucket of |u| by table: entry i holds the center (bf16, high half) and
+// the threshold count (low nibble) of the bf16 value with bits kLutBase + i.
+// |u| <= 0x3F81 (the block radius, rounded to bf16, is at least (1 - 2^-8.9)
+// of its largest value), and values below kLutBase share entry 0, which holds
+// unless a threshold lies in [0, kLutBase).
+constexpr uint32_t kLutBase = 0x3C00u;  // 2^-7
+constexpr int kLutSize = 0x3F90 - 0x3C00;
+constexpr int kEncWaves = 4;
+
+// A lane per key, a tile of 64 keys per wave (LDS: 4 tiles of 8 KiB and the
+// table).  Bound: VALU, ~3900 instructions per tile against ~11000 with a key
+// on 16 lanes; the block rows of the outputs ([16, seq]) are written as whole
+// runs of 64 tokens.  What saves the instructions, all with the same bits:
+//  * the butterfly runs in registers (7 per value; across 16 lanes every
+//    stage is a shuffle, a select and two adds);
+//  * bf16(x / d) for bf16 x and d is bf16(x * (1 / d)): the quotient of two
+//    8-bit significands is never within 2^-17 of a rounding boundary of 8
+//    bits unless it lies on one exactly, which only the subnormal range
+//    allows, where the product rounds to the quotient's own grid point;
+//  * x * x of a bf16 x is exact, so a multiply-add sums it (the multiply and
+//    the add are kept where the sum is small enough for products to underflow);
+//  * the bucket and its center are one table read instead of 14 compares and
+//    selects; sign bits and codes enter their words by align instructions.
+// Half rows at a time (8 KiB of LDS per wave) let three waves share a SIMD:
+// 134 us with whole rows and two.  8 x 131072 keys: 123 us (3.1 TB/s, VALU
+// ~85% busy) against 292 us on 16 lanes per key.
+__global__ __launch_bounds__(64 * kEncWaves, 3) void rabitq4_encode_kernel(const EncodeParams p, int tiles_per_bh,
+                                                                          int64_t n_tiles) {
+  // the table first: its reads then take their LDS offset as an immediate
+  __shared__ struct __attribute__((aligned(16))) {
+    uint32_t lut[kLutSize];
+    uint8_t tiles[kEncWaves][64 * 128];
+  } sm;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float thr[7], ctr[8];
+  bool table = true;
+#pragma unroll
+  for (int i = 0; i < 7; ++i) {
+    thr[i] = bf16_to_f32(p.thr[i]);
+    table = table && !(thr[i] >= 0.0f && thr[i] < __uint_as_float(kLutBase << 16));
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ctr[i] = bf16_to_f32(p.ctr[i]);
+  const int64_t tile = static_cast<int64_t>(blockIdx.x) * kEncWaves + wave;
+  const int64_t bh = tile / tiles_per_bh;
+  const int tok = 64 * static_cast<int>(tile - bh * tiles_per_bh);
+  if (!table) {  // (uniform)
+    if (tile < n_tiles) {
+      for (int i = 0; i < 64; i += 4) {
+        const int t = tok + i + (lane >> 4);
+        encode_key16(p, t < p.n ? bh * p.n + t : p.rows, lane & 15);
+      }
+    }
+    return;
+  }
+  for (int i = threadIdx.x; i < kLutSize; i += 64 * kEncWaves) {
+    const float u = __uint_as_float((kLutBase + i) << 16);
+    uint32_t tq = 0;
+#pragma unroll
+    for (int k = 0; k < 7; ++k) tq += u > thr[k] ? 1u : 0u;
+    float c = ctr[0];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) c = tq == static_cast<uint32_t>(k) ? ctr[k] : c;
+    sm.lut[i] = __float_as_uint(c) | tq;
+  }
+  __syncthreads();
+  if (tile >= n_tiles) return;
+  const int b = static_cast<int>(bh / p.kv), h = static_cast<int>(bh - static_cast<int64_t>(b) * p.kv);
+  uint8_t* const xt = sm.tiles[wave];
+  const int left = p.n - tok;
+  const uint16_t* const keys = p.keys + b * p.k_sb + h * p.k_sh + tok * p.k_st;
+
+  // ---- the row and its norm: block sums in order, then blocks b and b + 8, + 4, + 2, + 1 ----
+  float y[kDim];
+  float bs[kBlk];
+#pragma unroll
+  for (int c = 0; c < kBlk; ++c) {
+    if (c % 8 == 0) {  // half rows: 8 KiB of LDS per wave, three waves per SIMD
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the first half has been read
+      load_row_tile<8>(xt, keys + 8 * c, p.k_st, left);
+    }
+    const u32x4_t w = row_tile_chunk<8>(xt, lane, c % 8);
+    float s = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float lo = __uint_as_float(w[e] << 16), hi = __uint_as_float(w[e] & 0xFFFF0000u);
+      s = __builtin_fmaf(lo, lo, s);
+      s = __builtin_fmaf(hi, hi, s);
+      y[8 * c + 2 * e] = lo;
+      y[8 * c + 2 * e + 1] = hi;
+    }
+    bs[c] = s;
+  }
+  auto tree = [&]() {
+#pragma unroll
+    for (int d = 8; d >= 1; d >>= 1)
+#pragma unroll
+      for (int c = 0; c < d; ++c) bs[c] = bs[c] + bs[c + d];
+    return bs[0];
+  };
+  float ss = tree();
+  if (ss < kTinySum) {
+#pragma unroll
+    for (int c = 0; c < kBlk; ++c) {
+      float s = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s = s + y[8 * c + j] * y[8 * c + j];
+      bs[c] = s;
+    }
+    ss = tree();
+  }
+  const float knorm = bf16r(__builtin_sqrtf(ss));
+  const float rk = 1.0f / fmaxf(knorm, kBf16OneEm8);
+
+  // ---- unit row, signs, butterfly.  (+ 0 in the first stage leaves no -0, so
+  // none arises later: the sign bit of a y is y < 0.) ----
+  const uint32_t* sg = reinterpret_cast<const uint32_t*>(p.signs);
+#pragma unroll
+  for (int d = 0; d < kDim; d += 2) {
+    const uint32_t sp = sg[d >> 1];
+    const float s0 = __uint_as_float(sp << 16), s1 = __uint_as_float(sp & 0xFFFF0000u);
+    const float a = bf16r(y[d] * rk), c = bf16r(y[d + 1] * rk);
+    const float t = __builtin_fmaf(a, s0, 0.0f);
+    y[d] = __builtin_fmaf(c, s1, t);
+    y[d + 1] = __builtin_fmaf(-c, s1, t);
+  }
+#pragma unroll
+  for (int hh = 2; hh < kDim; hh <<= 1)
+#pragma unroll
+    for (int i = 0; i < kDim; ++i)
+      if (!(i & hh)) {
+        const float a = y[i], c = y[i + hh];
+        y[i] = a + c;
+        y[i + hh] = a - c;
+      }
+  // a NaN or an infinity in the row makes every y a NaN: sign bits and counts
+  // are then all 0 (the comparisons are false) and the weights NaN
+  uint32_t keep = ~0u;
+  if (!(y[0] == y[0])) {
+    keep = 0u;
+#pragma unroll
+    for (int d = 0; d < kDim; ++d) y[d] = 0.0f;
+  }
+
+  // ---- block radii ----
+  float rad[kBlk];
+  float least = INFINITY;
+  uint32_t near = ~0u;
+#pragma unroll
+  for (int c = 0; c < kBlk; ++c) {
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      y[8 * c + j] = bf16r(y[8 * c + j] * kHadScale);
+      s = __builtin_fmaf(y[8 * c + j], y[8 * c + j], s);
+    }
+    least = fminf(least, s);
+    // the hardware root (within 1 unit of the last place) rounds to the same
+    // bf16 as the exact one unless it lies within 2 units of a boundary
+    const float g = __builtin_amdgcn_sqrtf(s);
+    near = min(near, (__float_as_uint(g) - 0x7FFEu) << 16);
+    rad[c] = bf16r(g);
+  }
+  if (least < kTinySum || near <= 4u << 16) {
+#pragma unroll
+    for (int c = 0; c < kBlk; ++c) {
+      float s = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s = s + y[8 * c + j] * y[8 * c + j];
+      rad[c] = bf16r(__builtin_sqrtf(s));
+    }
+  }
+
+  // ---- blocks: direction, bucket, alpha, weight (PC:1170-1192) ----
+  if (lane >= left) return;
+  const uint32_t tt = p.t0 + tok + lane;
+  uint8_t* code_p = p.code + b * p.c_sb + h * p.c_sh;
+  uint32_t* packed_p = p.packed + b * p.p_sb + h * p.p_sh;
+  uint16_t* weight_p = p.weight + b * p.w_sb + h * p.w_sh;
+#pragma unroll
+  for (int blk = 0; blk < kBlk; ++blk) {
+    const float* v = y + 8 * blk;
+    // (within 2^-22 of 1 / d: see above)
+    const float r = __builtin_amdgcn_rcpf(fmaxf(rad[blk], kBf16OneEm8));
+    float alpha = 0.0f;
+    uint32_t packed = 0u, neg = 0u;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float au = bf16r(fabsf(v[j]) * r);
+      const uint32_t off = __builtin_elementwise_sub_sat(__float_as_uint(au), kLutBase << 16) >> 14;  // bytes
+      const uint32_t e = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(sm.lut) + off);
+      alpha = alpha + bf16r(__uint_as_float(e & 0xFFFF0000u) * au);
+      packed = __builtin_amdgcn_alignbit(e, packed, 4);  // count j to nibble j after the 8th
+    }
+#pragma unroll
+    for (int j = 7; j >= 0; --j) neg = __builtin_amdgcn_alignbit(neg, __float_as_uint(v[j]), 31);
+    const uint32_t code = ~neg & 0xFFu & keep;
+    uint32_t sp = code;  // bit j to bit 4 j
+    sp = (sp | sp << 12) & 0x000F000Fu;
+    sp = (sp | sp << 6) & 0x03030303u;
+    sp = (sp | sp << 3) & 0x11111111u;
+    packed = (packed & keep) | sp << 3;
+    alpha = fmaxf(alpha, 1e-6f);
+    const float w = bf16r((rad[blk] / alpha) * knorm);
+    (code_p + blk * p.c_sB)[tt] = static_cast<uint8_t>(code);
+    (packed_p + blk * p.p_sB)[tt] = packed;
+    (weight_p + blk * p.w_sB)[tt] = static_cast<uint16_t>(__float_as_uint(w) >> 16);
   }
 }
 
@@ -439,8 +657,20 @@ extern "C" int zkv_rabitq4_encode(const uint16_t* keys, int64_t k_sb, int64_t k_
   p.rows = static_cast<int64_t>(bs) * kv * n;
   const int64_t blocks = (p.rows * 16 + 255) / 256;
   ZKV_REQUIRE(blocks < (1ll << 31), "zkv_rabitq4_encode: too many rows (%lld)", static_cast<long long>(p.rows));
-  rabitq4_encode_kernel<<<static_cast<unsigned>(blocks), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(p);
-  return check_launch("rabitq4_encode_kernel");
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int tiles_per_bh = (n + 63) / 64;
+  const int64_t n_tiles = static_cast<int64_t>(bs) * kv * tiles_per_bh;
+  // A tile takes its wave ~11 us whatever it holds, and 3072 run at a time; 16
+  // lanes per key take ~0.25 us per 1000 keys over the whole chip.  8 heads of
+  // 1 / 4096 / 6144 / 16384 keys: 18.6 / 13.5 / 14.3 / 22.6 us by tiles, 3.5 /
+  // 11.2 / 18.1 / 41.8 us on 16 lanes (the last two with IEEE divisions).
+  if (p.rows >= 40960 && p.rows >= 48 * n_tiles) {
+    rabitq4_encode_kernel<<<static_cast<unsigned>((n_tiles + kEncWaves - 1) / kEncWaves), 64 * kEncWaves, 0, s>>>(
+        p, tiles_per_bh, n_tiles);
+    return check_launch("rabitq4_encode_kernel");
+  }
+  rabitq4_encode_small_kernel<<<static_cast<unsigned>(blocks), 256, 0, s>>>(p);
+  return check_launch("rabitq4_encode_small_kernel");
 }
 
 extern "C" int zkv_rabitq4_encode_query(const uint16_t* q, int64_t q_sr, int rows, const uint16_t* signs,

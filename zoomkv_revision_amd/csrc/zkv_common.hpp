@@ -176,33 +176,44 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N & 0x30) << 10) | 0x0F70);
 }
 
-// A wave's tile of 64 rows of 256 bytes (128 16-bit values) for kernels that
-// give each lane one whole row.  The rows come in as 16 coalesced DMAs of 4
-// rows; 16-byte chunk c of row r lands in slot c ^ (r & 15) of its row, so
-// that the 16 lanes of a read phase, each reading chunk c of its own row, hit
-// 16 different slots (all 64 banks once).  Row r < rows is at base + r *
-// stride (uint16 units, 16-byte aligned); rows past the end repeat the last.
-// Returns when the tile is there; only the wave itself reads it.
-constexpr int kRowTileBytes = 64 * 256;
+// A wave's tile of 64 rows of C 16-byte chunks (C = 16: whole rows of 128
+// 16-bit values, C = 8: half rows), for kernels that give each lane one row.
+// The rows come in as C coalesced DMAs of 1 KiB; chunk c of row r lands in
+// slot c ^ f(r) of its row, f(r) chosen so that the 16 lanes of a read phase,
+// each reading chunk c of its own row, hit every bank once.  Row r < rows is
+// at base + r * stride (uint16 units, 16-byte aligned); rows past the end
+// repeat the last.  Returns when the tile is there; only the wave itself
+// reads it.
+template <int C>
+__device__ __forceinline__ int row_tile_slot(int r, int c) {
+  static_assert(C == 16 || C == 8, "whole or half rows");
+  return c ^ ((C == 16 ? r : r >> 1) & (C - 1));
+}
+template <int C>
+__device__ __forceinline__ int row_tile_offset(int r, int c) {
+  return 16 * (C * r + row_tile_slot<C>(r, c));
+}
+template <int C>
 __device__ __forceinline__ void load_row_tile(uint8_t* tile, const uint16_t* base, int64_t stride, int rows) {
-  const int lane = threadIdx.x & 63, r0 = lane >> 4;
-  // chunk lane % 16 of row 4 i + r0 comes from chunk (lane ^ row) % 16
+  constexpr int kRows = 64 / C;  // per DMA
+  const int lane = threadIdx.x & 63, r0 = lane / C, slot = lane % C;
   if (rows >= 64) {
     const uint16_t* p = base + r0 * stride;
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      dma16(p + 4 * i * stride + 8 * ((lane ^ (4 * i + r0)) & 15), tile + 1024 * i);
+    for (int i = 0; i < C; ++i)
+      dma16(p + kRows * i * stride + 8 * row_tile_slot<C>(kRows * i + r0, slot), tile + 1024 * i);
   } else {
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      dma16(base + min(4 * i + r0, rows - 1) * stride + 8 * ((lane ^ (4 * i + r0)) & 15), tile + 1024 * i);
+    for (int i = 0; i < C; ++i)
+      dma16(base + min(kRows * i + r0, rows - 1) * stride + 8 * row_tile_slot<C>(kRows * i + r0, slot),
+            tile + 1024 * i);
   }
   wait_vmcnt<0>();
   asm volatile("" ::: "memory");
 }
-__device__ __forceinline__ int row_tile_offset(int r, int c) { return 256 * r + 16 * (c ^ (r & 15)); }
+template <int C>
 __device__ __forceinline__ u32x4_t row_tile_chunk(const uint8_t* tile, int r, int c) {
-  return *reinterpret_cast<const u32x4_t*>(tile + row_tile_offset(r, c));
+  return *reinterpret_cast<const u32x4_t*>(tile + row_tile_offset<C>(r, c));
 }
 
 // ---------------------------------------------------------------------------
