@@ -1,8 +1,10 @@
-"""The division step of the KIVI quantisation ladder (csrc/zkv_common.hpp,
-div_recip): q = x * r, r = 1 / b, then q + (x - q b) r with two fused
-multiply-adds.  For bf16 operands with normal quotients it must equal the
-IEEE fp32 division bit for bit, which the bit-exact pack and stage-2 kernels
-rely on (quant_pack.py's bf16 ladder, S:2003-2009).
+"""Divisions of the KIVI quantisation ladder (quant_pack.py's bf16 ladder,
+S:2003-2009).  The kernels need bf16(x / b) and take it as bf16(x * (1 / b))
+(csrc/zkv_common.hpp, kivi_code and kivi_scale; the last test here).  Where
+the fp32 quotient itself is wanted, the correction step of the other tests
+gives it: q = x * r, r = 1 / b, then q + (x - q b) r with two fused
+multiply-adds equals the IEEE fp32 division of bf16 operands bit for bit
+while the quotient is normal.
 
 In the normal range the rounding of every step depends only on the operands'
 significands (scaling x or b by a power of two scales every intermediate by
@@ -95,10 +97,17 @@ def _bf16_rne(x: np.ndarray) -> np.ndarray:
 
 
 def test_bf16_quotient_by_reciprocal_product():
-    """bf16(x / d) == bf16(x * (1 / d)) for bf16 x and d (rabitq4.hip's encode):
-    every pair of significands, with quotients from overflow down through
+    """bf16(x / d) == bf16(x * (1 / d)) for bf16 x and d (the KIVI ladder and
+    rabitq4.hip's encode): every bf16 x over 15 (signs, subnormals, infinities
+    and NaNs included), then every pair of significands, with quotients from overflow down through
     bf16's subnormal range, and with the reciprocal off by one unit in the
     last place (the hardware's) where the quotient is normal."""
+    x = _bf16_from_bits(np.arange(0x10000, dtype=np.uint32))
+    with np.errstate(invalid="ignore"):
+        by_product = _bf16_rne((x * np.float32(1.0 / 15.0)).astype(np.float32))
+        by_division = _bf16_rne(x / np.float32(15.0))
+    num = ~np.isnan(x)
+    assert np.array_equal(by_product[num], by_division[num])
     sig = 1.0 + np.arange(128, dtype=np.float64) / 128.0
     xs, ds = np.meshgrid(sig, sig, indexing="ij")
     for ex, ed in [(0, 0), (127, 0), (127, -1), (127, -26), (-60, 67), (100, 127), (-126, 0)] + \

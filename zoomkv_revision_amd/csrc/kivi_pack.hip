@@ -40,15 +40,9 @@ __global__ __launch_bounds__(128) void chunk_encode_kernel(
     mx = fmaxf(mx, x[t]);
     acc = acc + x[t];  // canonical sequential fp32 sum over the chunk's tokens
   }
-  const float safe = kivi_safe(kivi_scale(mn, mx));
-  if (safe < INFINITY) {
-    const float r = 1.0f / safe;
+  const float r = 1.0f / kivi_safe(kivi_scale(mn, mx));
 #pragma unroll
-    for (int t = 0; t < G; ++t) codes[t][d] = static_cast<uint8_t>(kivi_code_r(x[t], mn, safe, r));
-  } else {
-#pragma unroll
-    for (int t = 0; t < G; ++t) codes[t][d] = static_cast<uint8_t>(kivi_code(x[t], mn, safe));
-  }
+  for (int t = 0; t < G; ++t) codes[t][d] = static_cast<uint8_t>(kivi_code(x[t], mn, r));
 
   const int64_t bh = static_cast<int64_t>(b) * kv + h;
   const int64_t chunk = bh * n_chunks_max + chunk_start + c;
@@ -159,15 +153,9 @@ __global__ __launch_bounds__(128) void kivi4_pack_kernel(
       mx = fmaxf(mx, x[t]);
     }
     const float scale = kivi_scale(mn, mx);
-    const float safe = kivi_safe(scale);
-    if (safe < INFINITY) {
-      const float r = 1.0f / safe;
+    const float r = 1.0f / kivi_safe(scale);
 #pragma unroll
-      for (int t = 0; t < 32; ++t) kc[t][d] = static_cast<uint8_t>(kivi_code_r(x[t], mn, safe, r));
-    } else {
-#pragma unroll
-      for (int t = 0; t < 32; ++t) kc[t][d] = static_cast<uint8_t>(kivi_code(x[t], mn, safe));
-    }
+    for (int t = 0; t < 32; ++t) kc[t][d] = static_cast<uint8_t>(kivi_code(x[t], mn, r));
     const int p = d >> 3, j = d & 7;
     const int slot = 2 * (j & 3) + (j >> 2);
     uint16_t* km = k_meta + p * 16;
@@ -197,15 +185,9 @@ __global__ __launch_bounds__(128) void kivi4_pack_kernel(
       mx = fmaxf(mx, x[i]);
     }
     const float scale = kivi_scale(mn, mx);
-    const float safe = kivi_safe(scale);
-    if (safe < INFINITY) {
-      const float r = 1.0f / safe;
+    const float rs = 1.0f / kivi_safe(scale);
 #pragma unroll
-      for (int i = 0; i < 32; ++i) vc[t][32 * gd + i] = static_cast<uint8_t>(kivi_code_r(x[i], mn, safe, r));
-    } else {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) vc[t][32 * gd + i] = static_cast<uint8_t>(kivi_code(x[i], mn, safe));
-    }
+    for (int i = 0; i < 32; ++i) vc[t][32 * gd + i] = static_cast<uint8_t>(kivi_code(x[i], mn, rs));
     // token t = 16m + 4r + i: half m's block, entry (gd, r) = 4 scales then 4 zeros
     const int m = t >> 4, r = (t >> 2) & 3, i = t & 3;
     uint16_t* vm = v_meta + m * 128 + (gd * 4 + r) * 8;
