@@ -59,6 +59,22 @@ int zkv_chunk_encode(const uint16_t* keys, int64_t k_sb, int64_t k_sh, int64_t k
                      uint16_t* chunk_min, uint16_t* chunk_max, uint16_t* chunk_centroid,
                      uint8_t* chunk_valid, int32_t* packed_K, zkv_stream_t stream);
 
+/* A layer's prompt into the bf16 cache in one launch: of the source tokens of
+ * k / v (bf16 [bs, kv, sink + ret + local, 128] at element strides, rows
+ * 16-byte aligned), the first `sink` go to cache rows [sink_row, ..), the next
+ * `ret` to [ret_row, ..) and the last `local` to [local_row, ..) of k_rows /
+ * v_rows (bf16 [bs, kv, n_rows, 128] at strides (r_sb, r_sh), rows
+ * contiguous), and the ret / g complete chunks of the `ret` tokens' keys are
+ * encoded at chunk 0 as zkv_chunk_encode does (same outputs; g in {8, 16}).
+ * Replaces the row copies and the chunk encode of the reference's prefill
+ * (S:1009-1141), separate torch steps there. */
+int zkv_cache_prefill(const uint16_t* k, int64_t k_sb, int64_t k_sh, int64_t k_st, const uint16_t* v,
+                      int64_t v_sb, int64_t v_sh, int64_t v_st, int bs, int kv, int sink, int ret, int local,
+                      uint16_t* k_rows, uint16_t* v_rows, int64_t r_sb, int64_t r_sh, int n_rows, int sink_row,
+                      int ret_row, int local_row, int g, int n_chunks_max, uint16_t* chunk_min,
+                      uint16_t* chunk_max, uint16_t* chunk_centroid, uint8_t* chunk_valid, int32_t* packed_K,
+                      zkv_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * Format Q: 4-bit K (per channel, groups of 32 tokens) and V (per token,
  * groups of 32 channels) with fp16 scale / zero.  No reference counterpart

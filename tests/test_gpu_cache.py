@@ -187,6 +187,48 @@ def test_cache_offload_modes_identical(rng, monkeypatch):
         assert torch.equal(host.unified_values_cpu[l][:, :, :n], dev.unified_values[l][:, :, :n].cpu())
 
 
+@pytest.mark.parametrize("chunk,prompt,valid_start,rows", [
+    (16, 81, 0, 2),       # one retrieval token: no chunk
+    (16, 80 + 37, 3, 2),  # a second block of 2 tokens, a carry, left padding
+    (8, 80 + 64, 0, 2),   # whole blocks, no carry
+    (8, 80 + 95, 1, 2),   # a last block of 30 tokens: 3 chunks and a carry of 6
+    (16, 80 + 4001, 0, 1),  # one row of the batch at a time
+])
+def test_prefill_launch_writes_what_the_separate_steps_write(monkeypatch, chunk, prompt, valid_start, rows):
+    """The one-launch prefill of the bf16 device cache against the row copies
+    and chunk encode it replaces: every cache buffer, untouched rows included."""
+    from zoomkv_revision_amd import kivi
+    g = dict(L=1, bs=2, kv=3, hq=6, inp=4200, new=64, sink=16, local=64, interval=32, topk=32, thr=128)
+    gen = torch.Generator(device="cuda").manual_seed(prompt)
+    k, v = (torch.randn(2, prompt, 3, 128, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    k[0, prompt // 2, 0, 5], k[1, prompt // 2, 1, 7], k[0, prompt // 2, 2] = float("inf"), float("nan"), -0.0
+
+    def filled(one_launch):
+        cache, _ = _make(monkeypatch, chunk, 0.4, 0.3, chunk, chunk, storage="device", **g)
+        cache.valid_start = [valid_start] * 2
+        for t in (cache.unified_keys[0], cache.unified_values[0], cache._chunk_carry_keys[0]):
+            t.fill_(7.0)
+        if not one_launch:
+            monkeypatch.setattr(kivi, "cache_prefill_takes", lambda *t: False)
+        for b in range(0, 2, rows):
+            cache.prefill_update_kv_cache(None, k[b:b + rows], v[b:b + rows], 0, b)
+        monkeypatch.undo()
+        state = (cache.current_seq_len, cache.cpu_valid_end, cache._chunk_valid_end, cache._chunk_carry_count,
+                 cache.context)
+        return state, [cache.unified_keys[0], cache.unified_values[0], cache._chunk_key_min_gpu[0],
+                       cache._chunk_key_max_gpu[0], cache._chunk_key_centroid_gpu[0], cache._chunk_valid_mask_gpu[0],
+                       cache.key_kivi_packed_gpu[0], cache._chunk_carry_keys[0]]
+
+    (sa, a), (sb, b) = filled(True), filled(False)
+    assert sa == sb
+    for x, y in zip(a, b):
+        if x.dtype == torch.bfloat16:
+            nan = torch.isnan(y)
+            assert torch.equal(torch.isnan(x), nan)
+            x, y = x.masked_fill(nan, 0).view(torch.int16), y.masked_fill(nan, 0).view(torch.int16)
+        assert torch.equal(x, y)
+
+
 def test_cache_module_is_selectable_by_name():
     """The runtime resolves importlib.import_module(name).polar_cache and
     filters its kwargs by the constructor signature (Z/model_hub/qwen.py:336-419)."""

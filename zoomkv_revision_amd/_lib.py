@@ -26,6 +26,8 @@ SZ = C.c_size_t
 SIGNATURES = {
     "zkv_last_error": (C.c_char_p, []),
     "zkv_version": (C.c_char_p, []),
+    "zkv_cache_prefill": (I32, [P, I64, I64, I64, P, I64, I64, I64, I32, I32, I32, I32, I32, P, P, I64, I64, I32,
+                                I32, I32, I32, I32, I32, P, P, P, P, P, P]),
     "zkv_chunk_encode": (I32, [P, I64, I64, I64, I32, I32, I32, I32, I32, I32,
                                P, P, P, P, P, P]),
     "zkv_kivi4_pack": (I32, [P, I64, I64, I64, P, I64, I64, I64, I32, I32, I32, I32, I32,

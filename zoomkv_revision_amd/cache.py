@@ -303,12 +303,39 @@ class polar_cache:
             self.current_seq_len[layer_idx] = n
             return
         local_len = seq_len - retrieval_end
-        K[rows, :, n0:n0 + self.sink_size] = kt[:, :, vs:sink_end].to(self.dtype)
-        V[rows, :, n0:n0 + self.sink_size] = vt[:, :, vs:sink_end].to(self.dtype)
-        K[rows, :, n0 + self.sink_size:n0 + self.sink_size + local_len] = kt[:, :, retrieval_end:seq_len].to(self.dtype)
-        V[rows, :, n0 + self.sink_size:n0 + self.sink_size + local_len] = vt[:, :, retrieval_end:seq_len].to(self.dtype)
-        kr = kt[:, :, retrieval_start:retrieval_end].to(self.dtype)
-        vr = vt[:, :, retrieval_start:retrieval_end].to(self.dtype)
+        # a prefill writes its rows' retrieval zone from offset 0: no earlier
+        # carry belongs to them (the reference's per-layer carry would leak the
+        # previous row's tail into a one-row prefill)
+        self._chunk_carry_count[layer_idx] = 0
+        kt, vt = kt[:, :, vs:], vt[:, :, vs:]
+        chunk = self.quest_chunk_size
+        if not (self._kivi4 or self.enable_offload) and kt.device == K.device and kt.shape == vt.shape \
+                and kt.shape[1] == self.kv_head and kivi.cache_prefill_takes(kt, vt):
+            # rows and chunk metadata in one launch; the carry is the tail
+            # _store_chunks would keep
+            self._check_chunk_capacity(layer_idx, retrieval_length // chunk)
+            n = kivi.cache_prefill(kt, vt, self.sink_size, local_len, K[rows], V[rows], n0, 0, n0 + self.sink_size,
+                                   chunk, self._chunk_key_min_gpu[layer_idx][rows],
+                                   self._chunk_key_max_gpu[layer_idx][rows],
+                                   self._chunk_key_centroid_gpu[layer_idx][rows],
+                                   self._chunk_valid_mask_gpu[layer_idx][rows],
+                                   self.key_kivi_packed_gpu[layer_idx][rows])
+            self._chunk_valid_end[layer_idx] = max(self._chunk_valid_end[layer_idx], n)
+            tail = retrieval_length - n * chunk
+            if tail:
+                end = self.sink_size + retrieval_length
+                self._chunk_carry_keys[layer_idx][rows, :, :tail].copy_(kt[:, :, end - tail:end])
+            self._chunk_carry_count[layer_idx] = tail
+            self.cpu_valid_end[layer_idx] = retrieval_length
+            self.current_seq_len[layer_idx] = seq_len - vs
+            return
+        end = self.sink_size + retrieval_length
+        K[rows, :, n0:n0 + self.sink_size] = kt[:, :, :self.sink_size].to(self.dtype)
+        V[rows, :, n0:n0 + self.sink_size] = vt[:, :, :self.sink_size].to(self.dtype)
+        K[rows, :, n0 + self.sink_size:n0 + self.sink_size + local_len] = kt[:, :, end:].to(self.dtype)
+        V[rows, :, n0 + self.sink_size:n0 + self.sink_size + local_len] = vt[:, :, end:].to(self.dtype)
+        kr = kt[:, :, self.sink_size:end].to(self.dtype)
+        vr = vt[:, :, self.sink_size:end].to(self.dtype)
         if self._kivi4:
             # complete groups to Format Q, the < 32-token rest to the tail rows
             ng = kivi.kivi4_pack(kr, vr, self._kivi4_view(layer_idx, rows), 0)
@@ -327,10 +354,6 @@ class polar_cache:
             V[rows, :, :retrieval_length] = vr
         self.cpu_valid_end[layer_idx] = retrieval_length
         self.current_seq_len[layer_idx] = seq_len - vs
-        # a prefill writes its rows' retrieval zone from offset 0: no earlier
-        # carry belongs to them (the reference's per-layer carry would leak the
-        # previous row's tail into a one-row prefill)
-        self._chunk_carry_count[layer_idx] = 0
         self._store_chunks(layer_idx, kr, 0, rows)
 
     def sync(self, layer_idx, batch_idx):

@@ -69,6 +69,51 @@ def chunk_encode(keys: torch.Tensor, chunk_size: int, chunk_start: int,
     return n
 
 
+def cache_prefill(keys: torch.Tensor, values: torch.Tensor, sink: int, local: int, k_rows: torch.Tensor,
+                  v_rows: torch.Tensor, sink_row: int, ret_row: int, local_row: int, chunk_size: int,
+                  chunk_min: torch.Tensor, chunk_max: torch.Tensor, chunk_centroid: torch.Tensor,
+                  chunk_valid: torch.Tensor, packed_K: torch.Tensor) -> int:
+    """A prompt into bf16 cache rows in one launch: of the n tokens of keys /
+    values [bs, kv, n, 128], the first ``sink`` and the last ``local`` go to rows
+    ``sink_row`` and ``local_row`` on of k_rows / v_rows [bs, kv, rows, 128]
+    (contiguous rows), the tokens between to rows ``ret_row`` on, and the latter's
+    complete chunks are encoded at chunk 0 as ``chunk_encode`` does (the metadata
+    tensors are its).  Returns the number of chunks.  Everything is bf16 and
+    16-byte aligned (``cache_prefill_takes``)."""
+    require_gpu(keys, values, k_rows, v_rows, chunk_min, chunk_max, chunk_centroid, chunk_valid, packed_K)
+    bs, kv, n, _ = keys.shape
+    ret = n - sink - local
+    if keys.shape != values.shape or ret < 0 or not cache_prefill_takes(keys, values):
+        raise ValueError("cache_prefill: bf16 keys / values of one shape with 16-byte aligned rows")
+    for name, t in (("k_rows", k_rows), ("v_rows", v_rows)):
+        _check_bf16(name, t)
+        if tuple(t.shape[:2]) != (bs, kv) or t.stride(3) != 1 or t.stride(2) != HEAD_DIM or t.stride() != k_rows.stride():
+            raise ValueError(f"{name} must be [bs, kv, rows, 128] with contiguous rows")
+    for name, t in (("chunk_min", chunk_min), ("chunk_max", chunk_max), ("chunk_centroid", chunk_centroid)):
+        _check_bf16(name, t)
+        if not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous")
+    if chunk_valid.dtype != torch.bool or packed_K.dtype != torch.int32:
+        raise TypeError("chunk_valid must be bool and packed_K int32")
+    n_max = chunk_min.shape[2]
+    if tuple(packed_K.shape) != (bs, kv, n_max, 16, chunk_size) or not packed_K.is_contiguous():
+        raise ValueError(f"packed_K must be contiguous [{bs}, {kv}, {n_max}, 16, {chunk_size}]; "
+                         f"got {tuple(packed_K.shape)}")
+    ks, vs, rs = keys.stride(), values.stride(), k_rows.stride()
+    check(lib().zkv_cache_prefill(
+        ptr(keys), ks[0], ks[1], ks[2], ptr(values), vs[0], vs[1], vs[2], bs, kv, sink, ret, local,
+        ptr(k_rows), ptr(v_rows), rs[0], rs[1], k_rows.shape[2], sink_row, ret_row, local_row, chunk_size, n_max,
+        ptr(chunk_min), ptr(chunk_max), ptr(chunk_centroid), ptr(chunk_valid), ptr(packed_K), stream_of(keys)))
+    return ret // chunk_size
+
+
+def cache_prefill_takes(*rows: torch.Tensor) -> bool:
+    """Whether ``cache_prefill`` reads these [bs, kv, n, 128] tensors in place."""
+    return all(t.dtype == torch.bfloat16 and t.is_cuda and t.shape[-1] == HEAD_DIM and t.stride(-1) == 1
+               and not any(s % 8 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0 and t.shape[2] < 2 ** 20
+               for t in rows)
+
+
 # ---------------------------------------------------------------------------
 # Format Q
 # ---------------------------------------------------------------------------
