@@ -171,6 +171,44 @@ def test_decode_linear_residual_and_silu_mul(M, K, F_):
     _bf16_close(h, res + (act.float() @ wo.float().T).to(torch.bfloat16), ulps=2.0)
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (1, 128, 16), (4, 384, 4099), (3, 640, 33000),        # the stream: a lone unit, a row tail, several units per wave
+    (2, 2688, 130), (4, 4352, 90),                        # x rows past the first request, a chunk that K ends inside
+    (5, 2560, 6144), (9, 2560, 4896),                     # 4 KiB blocks at and under the wide kernel's 6144
+    (6, 384, 33000), (16, 256, 98304), (12, 2688, 9000),  # its units passed over twice; 1, 2 and more chains
+    (8, 7680, 1700), (16, 4352, 2890),                    # x rows of 123 and 139 KB
+])
+def test_decode_linear_units_and_k_ranges(M, K, N):
+    """The row, unit and K counts where the kernel or its split changes, with
+    strided rows, the residual over several units and Inf in a row that only
+    its own output sees.  fp32 sums of K products: within one bf16 unit of the
+    fp32 product at the tensor's scale (two after a norm)."""
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    res = torch.randn(M, N, generator=g, device="cuda").to(torch.bfloat16)
+    nw = (torch.rand(K, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
+    y = (x.float() @ w.float().T).to(torch.bfloat16)
+    out = torch.full((M, N + 3), 7.0, dtype=torch.bfloat16, device="cuda")
+    ds.decode_linear(x, w, out[:, :N], residual=res)
+    _bf16_close(out[:, :N], res + y, ulps=2.0)
+    assert (out[:, N:] == 7.0).all()
+    xn = ds.rms_norm(x, nw, 1e-6)
+    yn = (xn.float() @ w.float().T).to(torch.bfloat16)
+    normed = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    ds.decode_linear(x, w, normed, norm_w=nw, eps=1e-6)
+    _bf16_close(normed, yn, ulps=2.0)
+    if N % 2 == 0:
+        for source, norm_w in ((y, None), (yn, nw)):
+            act = torch.empty(M, N // 2, dtype=torch.bfloat16, device="cuda")
+            ds.decode_linear(x, w, act, norm_w=norm_w, eps=1e-6, silu_mul=True)
+            _bf16_close(act, torch.nn.functional.silu(source[:, :N // 2]) * source[:, N // 2:], ulps=2.0)
+    w[N // 2, K - 1] = float("inf")
+    ds.decode_linear(x, w, normed)
+    bad = torch.arange(N, device="cuda") == N // 2
+    assert torch.isfinite(normed[:, ~bad]).all() and not torch.isfinite(normed[:, bad]).any()
+
+
 def test_decode_linear_rejects_bad_shapes():
     from zoomkv_revision_amd._lib import ZkvError
     x = torch.zeros(4, 200, dtype=torch.bfloat16, device="cuda")

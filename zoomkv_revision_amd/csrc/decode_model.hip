@@ -2,14 +2,11 @@
 // runtime's layer_decode, Z/model_hub/LLM.py:208-251, with the rmsnorm /
 // rope / silu pieces of Z/model_hub/qwen.py:493-604):
 //
-//  * decode_linear_kernel: y[m, n] = sum_k x[m, k] * w[n, k] for the few rows
-//    m of a decode batch (M <= 16), bf16 in, fp32 accumulate, bf16 out, with
-//    an optional RMSNorm of x on the way in and an optional epilogue
-//    (residual add, or silu(gate) * up over the two halves of w).  The
-//    weights are streamed once from HBM: a workgroup owns 16 output rows, its
-//    waves split K, each k-block of 128 is four v_mfma_f32_16x16x32_bf16 with
-//    the 16 weight rows as A and the (normalised) x rows, staged in LDS, as
-//    the B columns.
+//  * decode_stream_kernel (M <= 4), decode_wide_kernel and decode_linear_kernel:
+//    y[m, n] = sum_k x[m, k] * w[n, k] for the few rows m of a decode batch
+//    (M <= 16), bf16 in, fp32 accumulate, bf16 out, with an optional RMSNorm of
+//    x on the way in and an optional epilogue (residual add, or silu(gate) * up
+//    over the two halves of w).  The weights stream once from HBM.
 //  * qk_norm_rope_kernel: per-head RMSNorm of q and k, rotate-half RoPE at
 //    one position, and the k / v rows written straight into the cache.
 //
@@ -18,8 +15,6 @@
 #include "zkv_common.hpp"
 
 #include <algorithm>
-#include <cstdio>
-#include <cstdlib>
 
 namespace zkv {
 namespace {
@@ -110,8 +105,8 @@ __device__ __forceinline__ void stage_x(const LinearParams& p, uint16_t* xs, flo
   __syncthreads();
 }
 
-// One workgroup per tile of 16 output rows (silu * up: 8 gate rows and the 8
-// matching up rows), NW waves splitting the K blocks.  Dynamic LDS: the M x K
+// M > 4, few tiles or no norm: one workgroup per tile of 16 output rows (silu *
+// up: 8 gate rows and the 8 matching up rows), NW waves splitting the K blocks.  Dynamic LDS: the M x K
 // bf16 input rows, then NW x 64 x 4 fp32 partial tiles.
 template <int kEpi, bool kNorm>
 __global__ __launch_bounds__(1024) void decode_linear_kernel(const LinearParams p) {
@@ -192,25 +187,257 @@ __global__ __launch_bounds__(1024) void decode_linear_kernel(const LinearParams 
   }
 }
 
+// Stages the M x K input rows into LDS (row stride ld elements), RMS-normalised:
+// bf16(x * rsqrt(mean(x^2) + eps) * w).  Wave w of nw takes rows w, w + nw, ...;
+// lane l holds 16-byte chunks l, l + 64, ... of a row, summed in that order.  load(), called ahead of the kernel's weight loads,
+// requests the first kChunks chunks of kRows rows per wave: a request behind the
+// weights waits for them.  The caller synchronises after run().
+template <int kRows>
+struct NormStage {
+  static constexpr int kChunks = 5;  // per lane: K <= 2560 needs no later load
+  u32x4_t xv[kRows][kChunks], wv[kChunks];
+
+  __device__ __forceinline__ void load_row(const LinearParams& p, int r, int m, int lane) {
+    const u32x4_t* xr = reinterpret_cast<const u32x4_t*>(p.x + min(m, p.M - 1) * p.x_ld);
+#pragma unroll
+    for (int j = 0; j < kChunks; ++j) xv[r][j] = xr[min(lane + 64 * j, (p.K >> 3) - 1)];
+  }
+  __device__ __forceinline__ void load(const LinearParams& p, int wave, int nw, int lane) {
+    const int last = (p.K >> 3) - 1;
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) load_row(p, r, wave + r * nw, lane);
+#pragma unroll
+    for (int j = 0; j < kChunks; ++j)
+      wv[j] = reinterpret_cast<const u32x4_t*>(p.norm_w)[min(lane + 64 * j, last)];
+  }
+
+  static __device__ __forceinline__ float sum_sq(const u32x4_t v, float ss) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float lo = __uint_as_float(v[e] << 16), hi = __uint_as_float(v[e] & 0xFFFF0000u);
+      ss = ss + lo * lo;
+      ss = ss + hi * hi;
+    }
+    return ss;
+  }
+  static __device__ __forceinline__ u32x4_t normed(u32x4_t v, float r, const u32x4_t w) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float lo = bf16r((__uint_as_float(v[e] << 16) * r) * __uint_as_float(w[e] << 16));
+      const float hi = bf16r((__uint_as_float(v[e] & 0xFFFF0000u) * r) * __uint_as_float(w[e] & 0xFFFF0000u));
+      v[e] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
+    }
+    return v;
+  }
+
+  __device__ __forceinline__ void norm_row(const LinearParams& p, uint16_t* xs, int ld, int row, int m, int lane) {
+    const int kv8 = p.K >> 3;
+    const u32x4_t* xr = reinterpret_cast<const u32x4_t*>(p.x + m * p.x_ld);
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kChunks; ++j)
+      if (lane + 64 * j < kv8) ss = sum_sq(xv[row][j], ss);
+    for (int i = lane + 64 * kChunks; i < kv8; i += 64) ss = sum_sq(xr[i], ss);
+    // mean as the sum times 1/K (torch's mean), then rsqrt(mean + eps)
+    const float r = rsqrtf(wave_sum(ss) * (1.0f / static_cast<float>(p.K)) + p.eps);
+#pragma unroll
+    for (int j = 0; j < kChunks; ++j) {
+      const int i = lane + 64 * j;
+      if (i < kv8) *reinterpret_cast<u32x4_t*>(xs + m * ld + 8 * i) = normed(xv[row][j], r, wv[j]);
+    }
+    for (int i = lane + 64 * kChunks; i < kv8; i += 64)
+      *reinterpret_cast<u32x4_t*>(xs + m * ld + 8 * i) =
+          normed(xr[i], r, reinterpret_cast<const u32x4_t*>(p.norm_w)[i]);
+  }
+
+  __device__ __forceinline__ void run(const LinearParams& p, uint16_t* xs, int ld, int wave, int nw, int lane) {
+#pragma unroll
+    for (int row = 0; row < kRows; ++row)
+      if (wave + row * nw < p.M) norm_row(p, xs, ld, row, wave + row * nw, lane);
+    for (int m = wave + kRows * nw; m < p.M; m += nw) {
+      load_row(p, 0, m, lane);
+      norm_row(p, xs, ld, 0, m, lane);
+    }
+  }
+};
+
+// ---------------------------------------------------------------------------
+// M > 4 and many units: the tiles of decode_linear_kernel as one stream.  A
+// unit's K blocks of 128 k form kA * S chains: block kb belongs to chain kb %
+// (kA * S), each chain sums its blocks in order in one accumulator, and the
+// chains are added in order: decode_linear_kernel's sums (a chain is one of its
+// waves), whatever waves work on them.
+//
+// A workgroup of nw waves is nw / S groups; the S waves of a group share a
+// unit, wave `part` of it taking blocks part, part + S, ..., and group g of the
+// grid takes units g, g + (groups in the grid), ...  A block is four loads (4
+// KiB); each wave keeps four blocks in flight, across unit ends and from before
+// the x rows are staged.  The loads are the same on every path: one that some
+// path skips makes the compiler wait for the whole stream at each round (past
+// a wave's last block they re-read the start of an x row).
+//
+// The normalised x rows sit in LDS (16 bytes apart in their banks where there is
+// room).  Against a workgroup per unit, which stages the rows for every unit
+// and waits for them before its first weight load (us at M = 6 / 12 / 16):
+// qkv 13.5 / 15.6 / 20.3 -> 12.2 / 12.3 / 13.6, gate and up 31.1 / 50.5 / 84.3 ->
+// 22.1 / 23.7 / 24.5, head 195 / 312 / 587 -> 142 / 148 / 152.
+// ---------------------------------------------------------------------------
+template <int kEpi, int kA>
+__global__ __launch_bounds__(512) void decode_wide_kernel(const LinearParams p, int n_units, int S, int xs_ld) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  constexpr int kDepth = 4;  // blocks in flight; a multiple of kA
+  uint16_t* xs = reinterpret_cast<uint16_t*>(lds);
+  const int M = p.M, K = p.K, N = p.N;
+  float4_t* red = reinterpret_cast<float4_t*>(lds + static_cast<size_t>(M) * xs_ld * 2);
+  const int nw = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 15, g = lane >> 4;
+  const int groups = nw / S, part = wave % S;
+  const int u0 = blockIdx.x * groups + wave / S, stride = gridDim.x * groups;
+  // every group of the workgroup passes the same number of unit ends (the
+  // barriers below); units past the end store nothing
+  const int n_iter = (n_units - 1 - static_cast<int>(blockIdx.x) * groups) / stride + 1;
+  const int cnt = (K / kLinKBlock - part + S - 1) / S;  // this wave's blocks of a unit
+  const int rounds = (cnt + kDepth - 1) / kDepth;       // kDepth blocks each, the last with some left out
+  const int n_rounds = n_iter * rounds;
+  const bool col_ok = c < M;
+
+  // row r of unit u as a row of w (rows past N repeat the last; not stored)
+  auto weight_row = [&](int u, int r) {
+    if constexpr (kEpi == kEpiSiluMul)
+      return min(8 * u + (r & 7), (N >> 1) - 1) + (r < 8 ? 0 : N >> 1);
+    else
+      return min(16 * u + r, N - 1);
+  };
+  NormStage<3> stage;
+  stage.load(p, wave, nw, lane);
+  float res0[4];  // the first unit's residual: lane (c, g) ends with rows 4g + i of x row c
+  if constexpr (kEpi == kEpiResidual) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) res0[i] = bf16_to_f32(p.res[min(c, M - 1) * p.res_ld + weight_row(u0, 4 * g + i)]);
+  }
+  int lu = u0, li = 0;
+  const uint16_t* wp;
+  auto point = [&]() {
+    wp = lu < n_units ? p.w + static_cast<int64_t>(weight_row(lu, c)) * K + 8 * g : p.x + 8 * g;
+  };
+  point();
+  auto load_block = [&](u32x4_t (&a)[4]) {
+    const int k = lu < n_units ? (part + li * S) * kLinKBlock : 0;
+    const uint16_t* src = li < cnt ? wp + k : p.x + 8 * g;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const u32x4_t*>(src + 32 * j);
+    if (++li == rounds * kDepth) {
+      li = 0;
+      lu += stride;
+      point();
+    }
+  };
+  u32x4_t wr[kDepth][4];
+#pragma unroll
+  for (int d = 0; d < kDepth; ++d) load_block(wr[d]);
+
+  stage.run(p, xs, xs_ld, wave, nw, lane);
+  __syncthreads();
+
+  float4_t acc[kA] = {};
+  int u = u0, ci = 0;
+  auto unit_end = [&]() {
+    const int uu = u;
+    u += stride;
+    ci = 0;
+    float4_t s = acc[0];
+    if (S > 1) {
+      // chain i * S + part of this wave; the unit's chains in order
+      float4_t* mine = red + (wave - part) * (64 * kA) + lane;
+      if (uu != u0) __syncthreads();  // (the last unit's chains have been read)
+#pragma unroll
+      for (int i = 0; i < kA; ++i) mine[(i * S + part) * 64] = acc[i];
+#pragma unroll
+      for (int i = 0; i < kA; ++i) acc[i] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      __syncthreads();
+      if (part != 0) return;
+      s = mine[0];
+      for (int w = 1; w < kA * S; ++w) {
+        const float4_t t = mine[w * 64];
+        s[0] += t[0], s[1] += t[1], s[2] += t[2], s[3] += t[3];
+      }
+    } else {
+#pragma unroll
+      for (int i = 1; i < kA; ++i) s[0] += acc[i][0], s[1] += acc[i][1], s[2] += acc[i][2], s[3] += acc[i][3];
+#pragma unroll
+      for (int i = 0; i < kA; ++i) acc[i] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    if (uu >= n_units) return;
+    if constexpr (kEpi == kEpiSiluMul) {
+      // gate rows sit in g < 2, the matching up rows 32 lanes higher
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float up = __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(s[i]), __float_as_uint(s[i]),
+                                                                          false, false)[1]);
+        const int j = 8 * uu + 4 * g + i;
+        if (g >= 2 || !col_ok || j >= (N >> 1)) continue;
+        const float gt = bf16r(s[i]), uv = bf16r(up);
+        const float act = bf16r(gt / (1.0f + expf(-gt)));
+        store_y(p, c, j, bf16r(act * uv));
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = 16 * uu + 4 * g + i;
+        if (!col_ok || n >= N) continue;
+        float y = bf16r(s[i]);
+        if constexpr (kEpi == kEpiResidual)
+          y = bf16r((uu == u0 ? res0[i] : bf16_to_f32(p.res[c * p.res_ld + n])) + y);
+        store_y(p, c, n, y);
+      }
+    }
+  };
+  const uint16_t* xl = xs + min(c, M - 1) * xs_ld + 8 * g;
+  for (int t = 0; t < n_rounds; ++t) {
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) {
+      if (ci + d < cnt) {  // (uniform)
+        const uint16_t* xp = xl + (part + (ci + d) * S) * kLinKBlock;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[d % kA] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8v_t, wr[d][j]),
+              __builtin_bit_cast(bf16x8v_t, *reinterpret_cast<const u32x4_t*>(xp + 32 * j)), acc[d % kA], 0, 0, 0);
+      }
+      load_block(wr[d]);
+    }
+    ci += kDepth;
+    if (ci >= cnt) unit_end();
+  }
+}
+
 // ---------------------------------------------------------------------------
 // The same linear for M <= 4 input rows as a weight stream.  A unit of work
-// is kR weight rows over all of K (silu * up: kR / 2 gate rows and the
-// matching up rows); every wave takes units gw, gw + (waves in the grid), ...
-// and walks their (unit, 512-element chunk) items with two items in flight:
-// each item is kR loads of 1 KiB of one weight row (64 lanes x 16 B, whole
-// cache lines, nontemporal) and, without a norm, the x rows' 16 B.  With the
-// norm, the workgroup stages the normalised x rows in LDS once (the grid is
-// at most a few workgroups per CU, so the staging is amortised over many
-// units).  v_dot2_f32_bf16 accumulates w x x in fp32; at the unit's last
-// chunk the lanes' partial sums are reduce-scattered with shuffles and the
-// epilogue (that of decode_linear_kernel) runs by lane pairs.  Waves never
-// wait for each other after the staging.  (The MFMA tile of
-// decode_linear_kernel makes each load instruction touch 16 rows x 64 B and
-// splits K over waves of a 16-row tile.)
+// is 4 weight rows over all of K (silu * up: 2 gate rows and the matching up
+// rows); every wave takes units gw, gw + (waves in the grid), ... and walks
+// their (unit, 512-element chunk) items with two items in flight: each item is
+// 4 loads of 1 KiB of one weight row (64 lanes x 16 B, whole cache lines,
+// nontemporal) and, without a norm, the x rows' 16 B.  The loads are the same
+// on every path, as in decode_wide_kernel.  With the norm, the workgroup stages
+// the normalised x rows in LDS once (the grid is at most a few workgroups per
+// CU, so the staging is amortised over many units), its x and norm-weight loads
+// ahead of the first weights.  v_dot2_f32_bf16 accumulates w x x in fp32; at
+// the unit's last chunk the lanes' partial sums are reduce-scattered with
+// shuffles and the epilogue (that of decode_linear_kernel) runs by lane
+// quadruples.  Waves never wait for each other after the staging.
+//
+// Bound: HBM, behind ~3 us of launch, first latency and last sums.  Qwen3-4B
+// projections at M = 4, cold weights, us: a plain read of the weights / with
+// loads that some paths skipped (and so every round waiting for all of them) /
+// now: qkv 6.6 / 11.6 / 8.7, o 5.2 / 7.9 / 6.9, gate and up 17.1 / 21.1 / 17.8,
+// down 9.2 / 13.1 / 13.0, head 120 / 122 / 119.  Units of 8 rows: 9.2, 7.2, 20.9,
+// 14.1, 126; of 2 rows: 8.6, 7.1, 18.1, 13.9, 125.
 // ---------------------------------------------------------------------------
 constexpr int kGemvMaxM = 4;
 constexpr int kGemvChunk = 512;  // elements of one row read by one wave instruction
 constexpr int kGemvWaves = 4;
+constexpr int kGemvRows = 4;     // weight rows per unit
 
 typedef __bf16 bf16x2v_t __attribute__((ext_vector_type(2)));
 
@@ -242,38 +469,26 @@ __device__ __forceinline__ void rs_step(const float (&v)[N], float (&o)[N / 2], 
   }
 }
 
-// The sum over the 64 lanes of value idx(lane) = lane >> (6 - log2 kV) of
-// the kV per-lane values (lanes equal in the high bits hold copies).
-template <int kV>
-__device__ __forceinline__ float lane_reduce(const float (&acc)[kV], int lane) {
-  float s;
-  if constexpr (kV == 32) {
-    float a[16], b[8], c[4], d[2], e[1];
-    rs_step<32>(acc, a, lane, 32);
-    rs_step<16>(a, b, lane, 16);
-    rs_step<8>(b, c, lane, 8);
-    rs_step<4>(c, d, lane, 4);
-    rs_step<2>(d, e, lane, 2);
-    s = e[0] + __shfl_xor(e[0], 1);
-  } else if constexpr (kV == 16) {
-    float a[8], b[4], c[2], d[1];
-    rs_step<16>(acc, a, lane, 32);
-    rs_step<8>(a, b, lane, 16);
-    rs_step<4>(b, c, lane, 8);
-    rs_step<2>(c, d, lane, 4);
-    s = d[0] + __shfl_xor(d[0], 2);
-    s = s + __shfl_xor(s, 1);
-  } else {
-    static_assert(kV == 8, "kV is 8, 16 or 32");
-    float a[4], b[2], c[1];
-    rs_step<8>(acc, a, lane, 32);
-    rs_step<4>(a, b, lane, 16);
-    rs_step<2>(b, c, lane, 8);
-    s = c[0] + __shfl_xor(c[0], 4);
-    s = s + __shfl_xor(s, 2);
-    s = s + __shfl_xor(s, 1);
-  }
-  return s;
+// The sum over the 64 lanes of value lane / 4 of the 16 per-lane values.
+__device__ __forceinline__ float lane_reduce(const float (&acc)[16], int lane) {
+  float a[8], b[4], c[2], d[1];
+  rs_step<16>(acc, a, lane, 32);
+  rs_step<8>(a, b, lane, 16);
+  rs_step<4>(b, c, lane, 8);
+  rs_step<2>(c, d, lane, 4);
+  float s = d[0] + __shfl_xor(d[0], 2);
+  return s + __shfl_xor(s, 1);
+}
+
+// 16 bytes of global memory at a wave-uniform base plus a lane's element
+// offset, not kept in the caches.  The base is opaque to the compiler: a load
+// from a choice of two stays one load instead of one per branch.
+__device__ __forceinline__ u32x4_t stream_load(const uint16_t* base, int off) {
+  typedef const __attribute__((address_space(1))) uint16_t* gptr_t;
+  typedef const __attribute__((address_space(1))) u32x4_t* gptr16_t;
+  uint64_t a = reinterpret_cast<uint64_t>(base);
+  asm("" : "+s"(a));
+  return __builtin_nontemporal_load(reinterpret_cast<gptr16_t>(reinterpret_cast<gptr_t>(a) + off));
 }
 
 // kSplit: the narrow projections.  A unit is then worked by the whole
@@ -281,15 +496,15 @@ __device__ __forceinline__ float lane_reduce(const float (&acc)[kV], int lane) {
 // launcher uses it for K >= 4 chunks), and the waves' partial sums meet in
 // LDS at the unit's end; the workgroups take units blockIdx.x, blockIdx.x +
 // gridDim.x, ...
-template <int kEpi, bool kNorm, int kR, int kD, bool kSplit>
+template <int kEpi, bool kNorm, bool kSplit>
 __global__ __launch_bounds__(64 * kGemvWaves) void decode_stream_kernel(const LinearParams p, int n_units) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  constexpr int kV = kR * kGemvMaxM;  // values per lane: acc[r * 4 + m]
-  constexpr int kShift = kV == 32 ? 1 : (kV == 16 ? 2 : 3);
-  float* rnorm = reinterpret_cast<float*>(lds);  // [4] norm factors
-  float* red = rnorm + kGemvMaxM;                // kSplit: [waves][64] partial sums
-  uint16_t* xs = reinterpret_cast<uint16_t*>(lds + 16 + (kSplit ? kGemvWaves * 64 * 4 : 0));  // normalised x [M][K]
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  constexpr int kR = kGemvRows, kD = 2;  // rows per unit, items in flight
+  constexpr int kV = kR * kGemvMaxM;     // values per lane: acc[r * 4 + m]
+  constexpr int kShift = 2;              // lanes 4 i .. 4 i + 3 end with value i
+  float* red = reinterpret_cast<float*>(lds);  // kSplit: [waves][64] partial sums
+  uint16_t* xs = reinterpret_cast<uint16_t*>(lds + (kSplit ? kGemvWaves * 64 * 4 : 0));  // normalised x [M][K]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int M = p.M, K = p.K, N = p.N;
   const int n_chunks = (K + kGemvChunk - 1) / kGemvChunk;
   // this wave's units u0, u0 + du, ... and chunks c0, c0 + dc, ... (cnt per unit)
@@ -299,98 +514,60 @@ __global__ __launch_bounds__(64 * kGemvWaves) void decode_stream_kernel(const Li
   const int cnt = kSplit ? (n_chunks - wave + kGemvWaves - 1) / kGemvWaves : n_chunks;
   const int n_my = u0 < n_units ? (n_units - 1 - u0) / du + 1 : 0;
   const int n_items = n_my * cnt;
-  constexpr int kXv = kGemvMaxM;  // the x rows' 16 B (no norm)
 
+  // weight row r of a unit (rows past N repeat the last one; not stored)
   auto unit_row = [&](int u, int r) {
     if constexpr (kEpi == kEpiSiluMul) {
-      const int half = N >> 1, j = u * (kR / 2) + (r % (kR / 2));
-      return j < half ? (r < kR / 2 ? j : half + j) : -1;
+      const int half = N >> 1, j = min(u * (kR / 2) + (r % (kR / 2)), half - 1);
+      return r < kR / 2 ? j : half + j;
     } else {
-      const int n = u * kR + r;
-      return n < N ? n : -1;
+      return min(u * kR + r, N - 1);
     }
   };
-  // item t of this wave: unit u0 + (t / cnt) du, chunk c0 + (t % cnt) dc
-  auto load_item = [&](int t, u32x4_t (&wv)[kR], u32x4_t (&xv)[kXv]) {
-    const int u = u0 + (t / cnt) * du, ci = c0 + (t % cnt) * dc;
-    const int k = ci * kGemvChunk + 8 * lane;
-    const bool ok = t < n_items && k < K;
+  NormStage<1> stage;
+  if constexpr (kNorm) stage.load(p, wave, kGemvWaves, lane);
+  // the first unit's residual (of the lane that stores it)
+  const int o_idx = lane >> kShift, o_r = o_idx / kGemvMaxM, o_m = o_idx % kGemvMaxM;
+  float res0 = 0.0f;
+  if constexpr (kEpi == kEpiResidual)
+    res0 = bf16_to_f32(p.res[min(o_m, M - 1) * p.res_ld + unit_row(min(u0, n_units - 1), o_r)]);
+
+  // past the wave's last item the loads re-read the first x row's start;
+  // lanes past K re-read the row's last 16 bytes (zeroed before use)
+  int lu = u0, lc = c0, li = 0;
+  auto load_item = [&](u32x4_t (&wv)[kR], u32x4_t (&xv)[kGemvMaxM]) {
+    const bool ok = lu < n_units;
+    const int k = ok ? min(lc * kGemvChunk + 8 * lane, K - 8) : 8 * (lane & 15);
 #pragma unroll
-    for (int r = 0; r < kR; ++r) {
-      const int row = unit_row(u, r);
-      wv[r] = ok && row >= 0 ? __builtin_nontemporal_load(
-                                   reinterpret_cast<const u32x4_t*>(p.w + static_cast<int64_t>(row) * K + k))
-                             : u32x4_t{0u, 0u, 0u, 0u};
-    }
+    for (int r = 0; r < kR; ++r)
+      wv[r] = stream_load(ok ? p.w + static_cast<int64_t>(unit_row(lu, r)) * K : p.x, k);
     if constexpr (!kNorm) {
 #pragma unroll
       for (int m = 0; m < kGemvMaxM; ++m)
-        xv[m] = ok && m < M ? *reinterpret_cast<const u32x4_t*>(p.x + m * p.x_ld + k) : u32x4_t{0u, 0u, 0u, 0u};
+        xv[m] = *reinterpret_cast<const u32x4_t*>(p.x + min(m, M - 1) * p.x_ld + k);
     }
+    lc += dc;
+    if (++li == cnt) lu += du, lc = c0, li = 0;
   };
-  // kD register slots of items in flight
-  u32x4_t wr[kD][kR], xr[kD][kXv];
+  u32x4_t wr[kD][kR], xr[kD][kGemvMaxM];
 #pragma unroll
-  for (int d = 0; d < kD; ++d) load_item(d, wr[d], xr[d]);
+  for (int d = 0; d < kD; ++d) load_item(wr[d], xr[d]);
 
   if constexpr (kNorm) {
-    // wave m: the RMS factor of x row m; then the normalised rows to LDS
-    // (the first items' weight loads are in flight)
-    if (wave < M) {
-      const u32x4_t* xrow = reinterpret_cast<const u32x4_t*>(p.x + wave * p.x_ld);
-      float ss = 0.0f;
-      for (int i = lane; i < (K >> 3); i += 64) {
-        const u32x4_t v = xrow[i];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float lo = __uint_as_float(v[e] << 16), hi = __uint_as_float(v[e] & 0xFFFF0000u);
-          ss = ss + lo * lo;
-          ss = ss + hi * hi;
-        }
-      }
-      ss = wave_sum(ss);
-      if (lane == 0) rnorm[wave] = rsqrtf(ss * (1.0f / static_cast<float>(K)) + p.eps);
-    }
-    __syncthreads();
-    for (int i = tid; i < M * (K >> 3); i += 64 * kGemvWaves) {
-      const int m = i / (K >> 3), k8 = i - m * (K >> 3);
-      u32x4_t v = reinterpret_cast<const u32x4_t*>(p.x + m * p.x_ld)[k8];
-      const float r = rnorm[m];
-      const u32x4_t wv = reinterpret_cast<const u32x4_t*>(p.norm_w)[k8];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float lo = bf16r((__uint_as_float(v[e] << 16) * r) * __uint_as_float(wv[e] << 16));
-        const float hi = bf16r((__uint_as_float(v[e] & 0xFFFF0000u) * r) * __uint_as_float(wv[e] & 0xFFFF0000u));
-        v[e] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
-      }
-      reinterpret_cast<u32x4_t*>(xs)[i] = v;
-    }
+    stage.run(p, xs, K, wave, kGemvWaves, lane);
     __syncthreads();
   }
 
   float acc[kV];
 #pragma unroll
   for (int j = 0; j < kV; ++j) acc[j] = 0.0f;
-  auto step = [&](int t, const u32x4_t (&wv)[kR], const u32x4_t (&xv)[kXv]) {
-    const int ci = c0 + (t % cnt) * dc;
-    const int k = ci * kGemvChunk + 8 * lane;
-    u32x4_t xm[kGemvMaxM];
-#pragma unroll
-    for (int m = 0; m < kGemvMaxM; ++m) {
-      if constexpr (kNorm)
-        xm[m] = m < M && k < K ? *reinterpret_cast<const u32x4_t*>(xs + m * K + k) : u32x4_t{0u, 0u, 0u, 0u};
-      else
-        xm[m] = xv[m];
-    }
-#pragma unroll
-    for (int r = 0; r < kR; ++r)
-#pragma unroll
-      for (int m = 0; m < kGemvMaxM; ++m) acc[r * kGemvMaxM + m] = dot8(wv[r], xm[m], acc[r * kGemvMaxM + m]);
-    if (t % cnt != cnt - 1) return;
-    // this wave's last chunk of the unit: sums over the lanes (and, split,
-    // over the waves), epilogue, fresh accumulators
-    const int u = u0 + (t / cnt) * du;
-    float s = lane_reduce<kV>(acc, lane);
+  int cu = u0, cc = c0, ci = 0;
+  // this wave's last chunk of a unit: sums over the lanes (and, split, over
+  // the waves), epilogue, fresh accumulators
+  auto unit_end = [&]() {
+    const int u = cu;
+    cu += du, cc = c0, ci = 0;
+    float s = lane_reduce(acc, lane);
 #pragma unroll
     for (int j = 0; j < kV; ++j) acc[j] = 0.0f;
     if constexpr (kSplit) {
@@ -403,32 +580,61 @@ __global__ __launch_bounds__(64 * kGemvWaves) void decode_stream_kernel(const Li
       __syncthreads();  // red is free for the next unit
       if (wave != 0) return;
     }
-    const int idx = lane >> kShift, r = idx / kGemvMaxM, m = idx % kGemvMaxM;
     const bool lead = (lane & ((1 << kShift) - 1)) == 0;
-    const int row = unit_row(u, r);
     if constexpr (kEpi == kEpiSiluMul) {
       // the up row of gate row r sits kR / 2 rows (32 lanes) higher
       const float up = __shfl_xor(s, 32);
-      if (lane >= 32 || !lead || m >= M || row < 0) return;
+      const int row = u * (kR / 2) + o_r;
+      if (lane >= 32 || !lead || o_m >= M || row >= (N >> 1)) return;
       const float gt = bf16r(s), uv = bf16r(up);
       const float act = bf16r(gt / (1.0f + expf(-gt)));
-      store_y(p, m, row, bf16r(act * uv));
+      store_y(p, o_m, row, bf16r(act * uv));
     } else {
-      if (!lead || m >= M || row < 0) return;
+      const int row = u * kR + o_r;
+      if (!lead || o_m >= M || row >= N) return;
       float y = bf16r(s);
-      if constexpr (kEpi == kEpiResidual) y = bf16r(bf16_to_f32(p.res[m * p.res_ld + row]) + y);
-      store_y(p, m, row, y);
+      if constexpr (kEpi == kEpiResidual)
+        y = bf16r((u == u0 ? res0 : bf16_to_f32(p.res[o_m * p.res_ld + row])) + y);
+      store_y(p, o_m, row, y);
     }
   };
-  // slot d holds items d, d + kD, ...: refilled kD items ahead (every slot
-  // index static)
-  for (int t = 0; t < n_items; t += kD) {
+  auto step = [&](u32x4_t (&wv)[kR], u32x4_t (&xv)[kGemvMaxM]) {
+    const int k = cc * kGemvChunk + 8 * lane;
+    if constexpr (kNorm) {
+#pragma unroll
+      for (int m = 0; m < kGemvMaxM; ++m)
+        xv[m] = *reinterpret_cast<const u32x4_t*>(xs + min(m, M - 1) * K + min(k, K - 8));
+    }
+    if (cc * kGemvChunk + kGemvChunk > K) {  // (uniform) the chunk ends inside the wave
+      const u32x4_t zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int r = 0; r < kR; ++r) wv[r] = k < K ? wv[r] : zero;
+#pragma unroll
+      for (int m = 0; m < kGemvMaxM; ++m) xv[m] = k < K ? xv[m] : zero;
+    }
+#pragma unroll
+    for (int r = 0; r < kR; ++r)
+#pragma unroll
+      for (int m = 0; m < kGemvMaxM; ++m)
+        acc[r * kGemvMaxM + m] = dot8(wv[r], xv[m], acc[r * kGemvMaxM + m]);
+    cc += dc;
+  };
+  // rounds of kD items, refilled while there is a round to refill for, then the
+  // last round alone
+  int t = 0;
+  for (; t + kD < n_items; t += kD) {
 #pragma unroll
     for (int d = 0; d < kD; ++d) {
-      if (t + d < n_items) {
-        step(t + d, wr[d], xr[d]);
-        load_item(t + d + kD, wr[d], xr[d]);
-      }
+      step(wr[d], xr[d]);
+      load_item(wr[d], xr[d]);
+      if (++ci == cnt) unit_end();
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < kD; ++d) {
+    if (t + d < n_items) {
+      step(wr[d], xr[d]);
+      if (++ci == cnt) unit_end();
     }
   }
 }
@@ -504,101 +710,99 @@ extern "C" int zkv_decode_linear(const uint16_t* x, int64_t x_ld, int M, int K, 
                   (norm_w == nullptr || (reinterpret_cast<uintptr_t>(norm_w) & 15) == 0),
               "zkv_decode_linear: x, w and the norm weight need 16-byte aligned rows");
   const size_t x_bytes = static_cast<size_t>(M) * K * 2;
+  // units of 16 weight rows (silu * up: 8 gate and 8 up)
   const int n_tiles = epilogue == kEpiSiluMul ? (N / 2 + 7) / 8 : (N + 15) / 16;
-  // waves per workgroup: enough resident waves to keep the weight stream busy
+  // waves per tile of decode_linear_kernel: enough resident waves to keep the
+  // weight stream busy, and few enough blocks per wave that its loads overlap.
+  // The x rows and 1 KiB for each of these waves fit the LDS
   const int nkb = K / kLinKBlock;
   int nw = 1;
   while (nw < 16 && nw * 2 <= nkb && static_cast<int64_t>(n_tiles) * nw < 4096) nw *= 2;
-  // and few enough k-blocks per wave that its loads overlap (the waves of a large N)
   while (nw < 16 && (nkb + nw - 1) / nw > 6) nw *= 2;
-  const size_t lds = x_bytes + static_cast<size_t>(nw) * 64 * 16;
-  ZKV_REQUIRE(lds <= 160 * 1024, "zkv_decode_linear: M x K = %d x %d needs %zu bytes of LDS (limit 160 KiB)", M,
-              K, lds);
+  ZKV_REQUIRE(x_bytes + static_cast<size_t>(nw) * 1024 <= 160 * 1024,
+              "zkv_decode_linear: M x K = %d x %d needs %zu bytes of LDS (limit 160 KiB)", M, K,
+              x_bytes + static_cast<size_t>(nw) * 1024);
   LinearParams p{x, x_ld, w, norm_w, eps, residual, res_ld, out, out_ld, M, K, N, out_f32};
   auto s = reinterpret_cast<hipStream_t>(stream);
-  if (M <= kGemvMaxM && !getenv("ZKV_LINEAR_MFMA")) {
-    // the weight stream: units of 8 rows for the wide projections, 4 or 2
-    // for narrower ones (at least ~2048 units); a few workgroups per CU
-    const int rows = epilogue == kEpiSiluMul ? N / 2 : N;
-    const int n_chunks = (K + kGemvChunk - 1) / kGemvChunk;
-    // narrow projections (fewer rows than ~2 units per wave of a full chip)
-    // split K over the waves of a workgroup
-    // (QKV, 6144 rows: 4 rows per unit 11.7 us, 2 rows 12.4; two or four
-    // items in flight per wave: the same or slower at every projection)
-    bool split = rows < 8192 && n_chunks >= kGemvWaves && !norm_w;
-    int R = split ? 4 : (rows >= 16384 ? 8 : (rows >= 4096 ? 4 : 2));
-    // ZKV_GEMV_SHAPE=R[,s] overrides the shape for tuning sweeps (s: split K)
-    if (const char* e = getenv("ZKV_GEMV_SHAPE")) {
-      int r = 0;
-      char sp = 0;
-      if (sscanf(e, "%d,%c", &r, &sp) >= 1 && (r == 2 || r == 4 || r == 8)) {
-        R = r;
-        split = sp == 's' && !norm_w && R == 4;
-      }
-    }
-    const int per_unit = epilogue == kEpiSiluMul ? R / 2 : R;
-    const int n_units = (rows + per_unit - 1) / per_unit;
-    const int grid_g = std::max(1, std::min(split ? n_units : (n_units + kGemvWaves - 1) / kGemvWaves, 768));
-    const size_t lds_g = 16 + (split ? kGemvWaves * 64 * 4 : 0) + (norm_w ? x_bytes : 0);
-    ZKV_REQUIRE(lds_g <= 160 * 1024, "zkv_decode_linear: M x K = %d x %d needs %zu bytes of LDS", M, K, lds_g);
-#define ZKV_GEMV(E, NORM, RR, D, SPLIT)                                                               \
+  // dynamic LDS above 64 KiB has to be allowed per kernel (once)
+#define ZKV_LAUNCH(KERNEL, GRID, BLOCK, LDS, ...)                                                     \
   do {                                                                                                \
     static bool big_lds_set = false;                                                                  \
-    if (lds_g > 64 * 1024 && !big_lds_set) {                                                          \
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_stream_kernel<E, NORM, RR, D, SPLIT>), \
+    if ((LDS) > 64 * 1024 && !big_lds_set) {                                                          \
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&KERNEL),                                 \
                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) \
         return fail(ZKV_EINVAL, "zkv_decode_linear: cannot raise the LDS limit to 160 KiB");          \
       big_lds_set = true;                                                                             \
     }                                                                                                 \
-    decode_stream_kernel<E, NORM, RR, D, SPLIT><<<grid_g, 64 * kGemvWaves, lds_g, s>>>(p, n_units);   \
+    KERNEL<<<GRID, BLOCK, LDS, s>>>(__VA_ARGS__);                                                     \
   } while (0)
-#define ZKV_GEMV_R(E, NORM)                 \
-  do {                                      \
-    if (split)                              \
-      ZKV_GEMV(E, NORM, 4, 2, true);        \
-    else if (R == 8)                        \
-      ZKV_GEMV(E, NORM, 8, 2, false);       \
-    else if (R == 4)                        \
-      ZKV_GEMV(E, NORM, 4, 2, false);       \
-    else                                    \
-      ZKV_GEMV(E, NORM, 2, 2, false);       \
+#define ZKV_COMMA ,
+  if (M <= kGemvMaxM) {
+    // the weight stream; narrow projections (fewer rows than ~2 units per wave
+    // of a full chip) split K over the waves of a workgroup
+    const int rows = epilogue == kEpiSiluMul ? N / 2 : N;
+    const int n_chunks = (K + kGemvChunk - 1) / kGemvChunk;
+    const bool split = rows < 8192 && n_chunks >= kGemvWaves && !norm_w;
+    const int per_unit = epilogue == kEpiSiluMul ? kGemvRows / 2 : kGemvRows;
+    const int n_units = (rows + per_unit - 1) / per_unit;
+    const int grid = std::max(1, std::min(split ? n_units : (n_units + kGemvWaves - 1) / kGemvWaves, 768));
+    const size_t lds = (split ? kGemvWaves * 64 * 4 : 0) + (norm_w ? x_bytes : 0);
+#define ZKV_GEMV(E)                                                                                   \
+  do {                                                                                                \
+    if (norm_w)                                                                                       \
+      ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA true ZKV_COMMA false>, grid, 64 * kGemvWaves, lds, p, n_units); \
+    else if (split)                                                                                   \
+      ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA false ZKV_COMMA true>, grid, 64 * kGemvWaves, lds, p, n_units); \
+    else                                                                                              \
+      ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA false ZKV_COMMA false>, grid, 64 * kGemvWaves, lds, p, n_units); \
   } while (0)
-    if (norm_w) {
-      if (epilogue == kEpiNone) ZKV_GEMV_R(kEpiNone, true);
-      else if (epilogue == kEpiResidual) ZKV_GEMV_R(kEpiResidual, true);
-      else ZKV_GEMV_R(kEpiSiluMul, true);
-    } else {
-      if (epilogue == kEpiNone) ZKV_GEMV_R(kEpiNone, false);
-      else if (epilogue == kEpiResidual) ZKV_GEMV_R(kEpiResidual, false);
-      else ZKV_GEMV_R(kEpiSiluMul, false);
-    }
-#undef ZKV_GEMV_R
+    if (epilogue == kEpiNone) ZKV_GEMV(kEpiNone);
+    else if (epilogue == kEpiResidual) ZKV_GEMV(kEpiResidual);
+    else ZKV_GEMV(kEpiSiluMul);
 #undef ZKV_GEMV
     return check_launch("decode_stream_kernel");
   }
-  const dim3 grid(n_tiles), block(64 * nw);
-  // dynamic LDS above 64 KiB has to be allowed per kernel (once)
-#define ZKV_LIN(E, NORM)                                                                              \
-  do {                                                                                                \
-    static bool big_lds_set = false;                                                                  \
-    if (lds > 64 * 1024 && !big_lds_set) {                                                            \
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_linear_kernel<E, NORM>),          \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) \
-        return fail(ZKV_EINVAL, "zkv_decode_linear: cannot raise the LDS limit to 160 KiB");          \
-      big_lds_set = true;                                                                             \
-    }                                                                                                 \
-    decode_linear_kernel<E, NORM><<<grid, block, lds, s>>>(p);                                        \
+  if (norm_w && static_cast<int64_t>(n_tiles) * nkb >= 6144) {
+    // 24 MB of weights and more: a workgroup per tile against this stream, M = 6,
+    // 4096 x 1024 (2048 blocks) 5.9 and 6.6 us, 6144 x 2560 (7680) 13.5 and 12.2.
+    // The chains of a unit's sum (nw of them) on at most four accumulators per
+    // wave and the rest as waves; eight waves (six where a unit takes one) stage
+    // the rows.
+    const int per_wave = std::min(nw, 4), S = nw / per_wave;
+    int nwv = S == 1 ? 6 : 8;
+    // (one unit's chains always fit: the requirement above)
+    if (S > 1 && x_bytes + static_cast<size_t>(nwv) * per_wave * 1024 > 160 * 1024) nwv = S;
+    const size_t red_bytes = S > 1 ? static_cast<size_t>(nwv) * per_wave * 1024 : 0;
+    // x rows 16 bytes apart in their banks where the LDS holds the padding
+    const int xs_ld = x_bytes + M * 16 + red_bytes <= 160 * 1024 ? K + 8 : K;
+    const size_t lds = static_cast<size_t>(M) * xs_ld * 2 + red_bytes;
+    // (a stream per wave from 2048 units on: one workgroup per CU, M = 16 head
+    // 152 us against 167 with a workgroup per six units)
+    const int grid = std::min((n_tiles + nwv / S - 1) / (nwv / S), n_tiles >= 2048 ? 256 : 1 << 30);
+#define ZKV_WIDE(E)                                                                               \
+  do {                                                                                            \
+    if (per_wave == 4) ZKV_LAUNCH(decode_wide_kernel<E ZKV_COMMA 4>, grid, 64 * nwv, lds, p, n_tiles, S, xs_ld); \
+    else if (per_wave == 2) ZKV_LAUNCH(decode_wide_kernel<E ZKV_COMMA 2>, grid, 64 * nwv, lds, p, n_tiles, S, xs_ld); \
+    else ZKV_LAUNCH(decode_wide_kernel<E ZKV_COMMA 1>, grid, 64 * nwv, lds, p, n_tiles, S, xs_ld); \
   } while (0)
-  if (norm_w) {
-    if (epilogue == kEpiNone) ZKV_LIN(kEpiNone, true);
-    else if (epilogue == kEpiResidual) ZKV_LIN(kEpiResidual, true);
-    else ZKV_LIN(kEpiSiluMul, true);
-  } else {
-    if (epilogue == kEpiNone) ZKV_LIN(kEpiNone, false);
-    else if (epilogue == kEpiResidual) ZKV_LIN(kEpiResidual, false);
-    else ZKV_LIN(kEpiSiluMul, false);
+    if (epilogue == kEpiNone) ZKV_WIDE(kEpiNone);
+    else if (epilogue == kEpiResidual) ZKV_WIDE(kEpiResidual);
+    else ZKV_WIDE(kEpiSiluMul);
+#undef ZKV_WIDE
+    return check_launch("decode_wide_kernel");
   }
+  const size_t lds = x_bytes + static_cast<size_t>(nw) * 1024;
+#define ZKV_LIN(E)                                                                                     \
+  do {                                                                                                 \
+    if (norm_w) ZKV_LAUNCH(decode_linear_kernel<E ZKV_COMMA true>, n_tiles, 64 * nw, lds, p);          \
+    else ZKV_LAUNCH(decode_linear_kernel<E ZKV_COMMA false>, n_tiles, 64 * nw, lds, p);                \
+  } while (0)
+  if (epilogue == kEpiNone) ZKV_LIN(kEpiNone);
+  else if (epilogue == kEpiResidual) ZKV_LIN(kEpiResidual);
+  else ZKV_LIN(kEpiSiluMul);
 #undef ZKV_LIN
+#undef ZKV_COMMA
+#undef ZKV_LAUNCH
   return check_launch("decode_linear_kernel");
 }
 
