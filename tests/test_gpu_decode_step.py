@@ -177,6 +177,8 @@ def test_decode_linear_residual_and_silu_mul(M, K, F_):
     (5, 2560, 6144), (9, 2560, 4896),                     # 4 KiB blocks at and under the wide kernel's 6144
     (6, 384, 33000), (16, 256, 98304), (12, 2688, 9000),  # its units passed over twice; 1, 2 and more chains
     (8, 7680, 1700), (16, 4352, 2890),                    # x rows of 123 and 139 KB
+    (5, 2048, 2570), (16, 128, 4100), (6, 9728, 514),     # units of 11 rows, 9 and 3 (the last short); 5 K blocks or 4
+    (5, 14720, 34), (7, 1152, 1), (8, 3072, 18),          # 8 K blocks per wave or 7; one row; half of the waves with one
 ])
 def test_decode_linear_units_and_k_ranges(M, K, N):
     """The row, unit and K counts where the kernel or its split changes, with

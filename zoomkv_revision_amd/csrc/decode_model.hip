@@ -2,7 +2,8 @@
 // runtime's layer_decode, Z/model_hub/LLM.py:208-251, with the rmsnorm /
 // rope / silu pieces of Z/model_hub/qwen.py:493-604):
 //
-//  * decode_stream_kernel (M <= 4), decode_wide_kernel and decode_linear_kernel:
+//  * decode_stream_kernel (M <= 4), decode_rows_kernel, decode_wide_kernel and
+//    decode_linear_kernel:
 //    y[m, n] = sum_k x[m, k] * w[n, k] for the few rows m of a decode batch
 //    (M <= 16), bf16 in, fp32 accumulate, bf16 out, with an optional RMSNorm of
 //    x on the way in and an optional epilogue (residual add, or silu(gate) * up
@@ -58,57 +59,52 @@ __device__ __forceinline__ void store_y(const LinearParams& p, int m, int n, flo
     reinterpret_cast<uint16_t*>(p.out)[m * p.out_ld + n] = f32_to_bf16_bits(y);
 }
 
-// Stages the M x K input rows into LDS (xs), RMS-normalised when kNorm:
+// Stages the M x K input rows into LDS (xs), RMS-normalised:
 // bf16(x * rsqrt(mean(x^2) + eps) * w).  red: M floats of scratch.
-template <bool kNorm>
 __device__ __forceinline__ void stage_x(const LinearParams& p, uint16_t* xs, float* red) {
   const int nw = blockDim.x >> 6;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int M = p.M, K = p.K;
   const int kv8 = K >> 3;  // 16-byte chunks per row
-  if constexpr (kNorm) {
-    // wave m' reduces rows m = m', m' + nw, ... (fixed order: deterministic)
-    for (int m = wave; m < M; m += nw) {
-      const u32x4_t* xr = reinterpret_cast<const u32x4_t*>(p.x + m * p.x_ld);
-      float ss = 0.0f;
-      for (int i = lane; i < kv8; i += 64) {
-        const u32x4_t v = xr[i];
+  // wave m' reduces rows m = m', m' + nw, ... (fixed order: deterministic)
+  for (int m = wave; m < M; m += nw) {
+    const u32x4_t* xr = reinterpret_cast<const u32x4_t*>(p.x + m * p.x_ld);
+    float ss = 0.0f;
+    for (int i = lane; i < kv8; i += 64) {
+      const u32x4_t v = xr[i];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float lo = __uint_as_float(v[e] << 16), hi = __uint_as_float(v[e] & 0xFFFF0000u);
-          ss = ss + lo * lo;
-          ss = ss + hi * hi;
-        }
+      for (int e = 0; e < 4; ++e) {
+        const float lo = __uint_as_float(v[e] << 16), hi = __uint_as_float(v[e] & 0xFFFF0000u);
+        ss = ss + lo * lo;
+        ss = ss + hi * hi;
       }
-      // mean as the sum times 1/K (torch's mean), then rsqrt(mean + eps)
-      ss = wave_sum(ss);
-      if (lane == 0) red[m] = rsqrtf(ss * (1.0f / static_cast<float>(K)) + p.eps);
     }
-    __syncthreads();
+    // mean as the sum times 1/K (torch's mean), then rsqrt(mean + eps)
+    ss = wave_sum(ss);
+    if (lane == 0) red[m] = rsqrtf(ss * (1.0f / static_cast<float>(K)) + p.eps);
   }
+  __syncthreads();
   for (int i = tid; i < M * kv8; i += blockDim.x) {
     const int m = i / kv8, k8 = i - m * kv8;
     u32x4_t v = reinterpret_cast<const u32x4_t*>(p.x + m * p.x_ld)[k8];
-    if constexpr (kNorm) {
-      const float r = red[m];
-      const u32x4_t wv = reinterpret_cast<const u32x4_t*>(p.norm_w)[k8];
+    const float r = red[m];
+    const u32x4_t wv = reinterpret_cast<const u32x4_t*>(p.norm_w)[k8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float lo = bf16r((__uint_as_float(v[e] << 16) * r) * __uint_as_float(wv[e] << 16));
-        const float hi =
-            bf16r((__uint_as_float(v[e] & 0xFFFF0000u) * r) * __uint_as_float(wv[e] & 0xFFFF0000u));
-        v[e] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
-      }
+    for (int e = 0; e < 4; ++e) {
+      const float lo = bf16r((__uint_as_float(v[e] << 16) * r) * __uint_as_float(wv[e] << 16));
+      const float hi =
+          bf16r((__uint_as_float(v[e] & 0xFFFF0000u) * r) * __uint_as_float(wv[e] & 0xFFFF0000u));
+      v[e] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
     }
     reinterpret_cast<u32x4_t*>(xs)[i] = v;
   }
   __syncthreads();
 }
 
-// M > 4, few tiles or no norm: one workgroup per tile of 16 output rows (silu *
+// M > 4, few tiles, with a norm: one workgroup per tile of 16 output rows (silu *
 // up: 8 gate rows and the 8 matching up rows), NW waves splitting the K blocks.  Dynamic LDS: the M x K
 // bf16 input rows, then NW x 64 x 4 fp32 partial tiles.
-template <int kEpi, bool kNorm>
+template <int kEpi>
 __global__ __launch_bounds__(1024) void decode_linear_kernel(const LinearParams p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   uint16_t* xs = reinterpret_cast<uint16_t*>(lds);
@@ -117,7 +113,7 @@ __global__ __launch_bounds__(1024) void decode_linear_kernel(const LinearParams 
   const int c = lane & 15, g = lane >> 4;
   const int M = p.M, K = p.K;
   float* red = reinterpret_cast<float*>(lds + static_cast<size_t>(M) * K * 2);
-  stage_x<kNorm>(p, xs, red);
+  stage_x(p, xs, red);
 
   // ---- weight rows of this tile ----
   const int tile = blockIdx.x;
@@ -182,6 +178,125 @@ __global__ __launch_bounds__(1024) void decode_linear_kernel(const LinearParams 
       if (n >= p.N) continue;
       float y = bf16r(s[i]);
       if constexpr (kEpi == kEpiResidual) y = bf16r(bf16_to_f32(p.res[c * p.res_ld + n]) + y);
+      store_y(p, c, n, y);
+    }
+  }
+}
+
+// M > 4 without a norm (o, down): decode_linear_kernel's sums with nothing
+// staged.  The waves of a workgroup split the K blocks (wave w takes blocks w, w
+// + nw, ...), so each element of x is used by one wave: it comes from memory
+// (the L2) next to its weights, with no barrier before the first weight load.
+// A unit is R <= 16 output rows (silu * up: R <= 8 pairs): lanes of the A rows
+// past R repeat row R - 1, which moves no more memory, and a row's sum does not
+// depend on the unit it is in.
+//
+// Bound: HBM, behind launch, first latency and last sums.  Against a workgroup
+// per 16 rows that stages x in LDS (cold weights, us at M = 6): 2560 x 4096 (o) 9.1
+// -> 7.5, 2560 x 9728 (down) 17.1 -> 13.1 (R = 10: 256 units, not 160), 4096 x 12288
+// 24.8 -> 23.2, 1024 x 3072 6.5 -> 5.3; silu, 19456 x 2560, M = 16: 51.5 -> 29.0.
+// (151936 x 1024, which only a head without its norm would ask for: 58.8 -> 59.9
+// at M = 6, 109 -> 76 at M = 16.)
+
+// The sum over kCnt K blocks of a wave, three blocks of loads in flight.  The
+// barriers keep the loads where they are: left to itself the compiler sinks them
+// to their uses (down 13.1 -> 14.1 us).
+template <int kCnt>
+__device__ __forceinline__ float4_t row_blocks(const uint16_t* wr, const uint16_t* xr, int wave, int nw) {
+  constexpr int kDepth = kCnt < 3 ? kCnt : 3;  // blocks in flight
+  float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (kCnt > 0) {
+    u32x4_t a[kDepth][4], b[kDepth][4];
+    auto load_block = [&](int i) {
+      const int k = (wave + i * nw) * kLinKBlock;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[i % kDepth][j] = *reinterpret_cast<const u32x4_t*>(wr + k + 32 * j);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[i % kDepth][j] = *reinterpret_cast<const u32x4_t*>(xr + k + 32 * j);
+    };
+#pragma unroll
+    for (int i = 0; i < kDepth; ++i) load_block(i);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kCnt; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v_t, a[i % kDepth][j]),
+                                                      __builtin_bit_cast(bf16x8v_t, b[i % kDepth][j]), acc, 0, 0, 0);
+      if (i + kDepth < kCnt) load_block(i + kDepth);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  return acc;
+}
+
+template <int kEpi, int kCnt>
+__global__ __launch_bounds__(1024) void decode_rows_kernel(const LinearParams p, int R) {
+  __shared__ float4_t red[16 * 64];
+  const int nw = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 15, g = lane >> 4;
+  const int K = p.K, N = p.N;
+  const int nkb = K / kLinKBlock;
+  const bool col_ok = c < p.M;
+  const int n0 = blockIdx.x * R;
+  // row r of this unit as a row of w (rows past the unit or N repeat the last; not stored)
+  auto weight_row = [&](int r) {
+    if constexpr (kEpi == kEpiSiluMul)
+      return min(n0 + min(r & 7, R - 1), (N >> 1) - 1) + (r < 8 ? 0 : N >> 1);
+    else
+      return min(n0 + min(r, R - 1), N - 1);
+  };
+  const uint16_t* wr = p.w + static_cast<int64_t>(weight_row(c)) * K + 8 * g;
+  const uint16_t* xr = p.x + min(c, p.M - 1) * p.x_ld + 8 * g;
+  uint16_t res[4];  // lane (c, g) ends with rows 4g + i of x row c
+  if constexpr (kEpi == kEpiResidual) {
+    if (wave == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) res[i] = p.res[min(c, p.M - 1) * p.res_ld + weight_row(4 * g + i)];
+    }
+  }
+  // the wave's blocks are all there but for the last: a wave without it takes a
+  // straight line of its own (loading some other line in its place costs the load
+  // path as much as a block: 6144 x 2560 13.3 us, so 9.7)
+  const bool full = wave + (kCnt - 1) * nw < nkb;  // (uniform)
+  float4_t acc;
+  if (kCnt == 1 || full) {
+    asm volatile("; all blocks");  // (unlike the other branch's, so that the loads stay in theirs)
+    acc = row_blocks<kCnt>(wr, xr, wave, nw);
+  } else {
+    asm volatile("; one fewer");
+    acc = row_blocks<kCnt - 1>(wr, xr, wave, nw);
+  }
+
+  // ---- sum the waves' partial tiles in wave order, then the epilogue ----
+  red[wave * 64 + lane] = acc;
+  __syncthreads();
+  if (wave != 0) return;
+  float4_t s = red[lane];
+  for (int w = 1; w < nw; ++w) {
+    const float4_t t = red[w * 64 + lane];
+    s[0] += t[0], s[1] += t[1], s[2] += t[2], s[3] += t[3];
+  }
+  if constexpr (kEpi == kEpiSiluMul) {
+    // gate rows sit in g < 2, the matching up rows 32 lanes higher
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float up = __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(s[i]), __float_as_uint(s[i]),
+                                                                        false, false)[1]);
+      const int r = 4 * g + i, j = n0 + r;
+      if (g >= 2 || !col_ok || r >= R || j >= (N >> 1)) continue;
+      const float gt = bf16r(s[i]), u = bf16r(up);
+      const float act = bf16r(gt / (1.0f + expf(-gt)));
+      store_y(p, c, j, bf16r(act * u));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 4 * g + i, n = n0 + r;
+      if (!col_ok || r >= R || n >= N) continue;
+      float y = bf16r(s[i]);
+      if constexpr (kEpi == kEpiResidual) y = bf16r(bf16_to_f32(res[i]) + y);
       store_y(p, c, n, y);
     }
   }
@@ -791,16 +906,38 @@ extern "C" int zkv_decode_linear(const uint16_t* x, int64_t x_ld, int M, int K, 
 #undef ZKV_WIDE
     return check_launch("decode_wide_kernel");
   }
+  if (!norm_w) {
+    // rows (or pairs) per unit: the number of units is rounded up to whole rounds
+    // of 256 CUs (160 tiles of 16 rows leave 96 CUs idle: down at M = 6 17.1 us, in
+    // 256 units of 10 rows 13.1)
+    const int rows = epilogue == kEpiSiluMul ? N / 2 : N;
+    const int units = (n_tiles + 255) / 256 * 256;
+    const int R = (rows + units - 1) / units;
+    const int grid = (rows + R - 1) / R;
+    // at most 8 blocks per wave: the LDS requirement above bounds K at M >= 5
+    const int cnt = (nkb + nw - 1) / nw;
+#define ZKV_ROWS_CNT(E, C)                                                    \
+  case C:                                                                     \
+    decode_rows_kernel<E, C><<<grid, 64 * nw, 0, s>>>(p, R);                  \
+    break;
+#define ZKV_ROWS(E)                                                           \
+  switch (cnt) {                                                              \
+    ZKV_ROWS_CNT(E, 1) ZKV_ROWS_CNT(E, 2) ZKV_ROWS_CNT(E, 3) ZKV_ROWS_CNT(E, 4) \
+    ZKV_ROWS_CNT(E, 5) ZKV_ROWS_CNT(E, 6) ZKV_ROWS_CNT(E, 7) ZKV_ROWS_CNT(E, 8) \
+    default:                                                                  \
+      return fail(ZKV_EINVAL, "zkv_decode_linear: %d K blocks per wave", cnt); \
+  }
+    if (epilogue == kEpiNone) ZKV_ROWS(kEpiNone)
+    else if (epilogue == kEpiResidual) ZKV_ROWS(kEpiResidual)
+    else ZKV_ROWS(kEpiSiluMul)
+#undef ZKV_ROWS
+#undef ZKV_ROWS_CNT
+    return check_launch("decode_rows_kernel");
+  }
   const size_t lds = x_bytes + static_cast<size_t>(nw) * 1024;
-#define ZKV_LIN(E)                                                                                     \
-  do {                                                                                                 \
-    if (norm_w) ZKV_LAUNCH(decode_linear_kernel<E ZKV_COMMA true>, n_tiles, 64 * nw, lds, p);          \
-    else ZKV_LAUNCH(decode_linear_kernel<E ZKV_COMMA false>, n_tiles, 64 * nw, lds, p);                \
-  } while (0)
-  if (epilogue == kEpiNone) ZKV_LIN(kEpiNone);
-  else if (epilogue == kEpiResidual) ZKV_LIN(kEpiResidual);
-  else ZKV_LIN(kEpiSiluMul);
-#undef ZKV_LIN
+  if (epilogue == kEpiNone) ZKV_LAUNCH(decode_linear_kernel<kEpiNone>, n_tiles, 64 * nw, lds, p);
+  else if (epilogue == kEpiResidual) ZKV_LAUNCH(decode_linear_kernel<kEpiResidual>, n_tiles, 64 * nw, lds, p);
+  else ZKV_LAUNCH(decode_linear_kernel<kEpiSiluMul>, n_tiles, 64 * nw, lds, p);
 #undef ZKV_COMMA
 #undef ZKV_LAUNCH
   return check_launch("decode_linear_kernel");
