@@ -151,6 +151,30 @@ def test_encode_tiles_match_short_calls(bs, kv, n, t0, thresholds):
     assert torch.equal(got[1].view(torch.int16)[~nan], want[1].view(torch.int16)[~nan])
 
 
+def test_encode_tiles_round_to_minus_zero(rng):
+    """y rounds to -0 where a bf16-subnormal quotient is what two cancelling
+    entries leave: a -0 is not below zero, so its sign bit is 1 (y >= 0), in a
+    call of 40960 keys as in one of a few."""
+    zk = _zk()
+    n, special = 40964, 70
+    sg = np.where(rng.integers(0, 2, 128) == 1, 1.0, -1.0).astype(np.float32)
+    x = rng.standard_normal((n, 128)).astype(np.float32)
+    x[:special:3] = 0.0
+    for i in range(0, special, 3):
+        x[i, 0] = x[i, 1] = 1.0
+        x[i, 2 + i] = -3e-40
+    x = bf16r(x * sg)
+    _, y = r4.srht_unit(x[:special], sg)
+    assert (((y == 0) & np.signbit(y)).sum(axis=1)[::3] >= 32).all()
+    want = r4.encode_keys(x[:special], sg)
+    for keys in (x[None, None], x[None, None, :special]):
+        code, w, packed = zk.batch_encode(_bf16(keys), _bf16(sg), *_levels(zk))
+        torch.cuda.synchronize()
+        got = code[0, 0, :, :special].cpu().numpy(), packed[0, 0, :, :special].cpu().numpy(), _bits(w[0, 0, :, :special])
+        for a, b in zip(got, (want[0], want[1], bf16_bits(want[2]))):
+            assert np.array_equal(a, b)
+
+
 def test_query_blocks_match_oracle(rng):
     zk = _zk()
     sg = np.where(rng.integers(0, 2, 128) == 1, 1.0, -1.0).astype(np.float32)

@@ -19,6 +19,8 @@
 // and unit token stride.
 #include "zkv_common.hpp"
 
+#include <climits>
+
 namespace zkv {
 namespace {
 
@@ -275,8 +277,8 @@ __global__ __launch_bounds__(64 * kEncWaves, 3) void rabitq4_encode_kernel(const
   const float knorm = bf16r(__builtin_sqrtf(ss));
   const float rk = 1.0f / fmaxf(knorm, kBf16OneEm8);
 
-  // ---- unit row, signs, butterfly.  (+ 0 in the first stage leaves no -0, so
-  // none arises later: the sign bit of a y is y < 0.) ----
+  // ---- unit row, signs, butterfly.  (+ 0 in the first stage leaves no -0, and
+  // sums make none.) ----
   const uint32_t* sg = reinterpret_cast<const uint32_t*>(p.signs);
 #pragma unroll
   for (int d = 0; d < kDim; d += 2) {
@@ -309,6 +311,7 @@ __global__ __launch_bounds__(64 * kEncWaves, 3) void rabitq4_encode_kernel(const
   float rad[kBlk];
   float least = INFINITY;
   uint32_t near = ~0u;
+  int lowest = 0;  // of the y's bits: INT_MIN is -0
 #pragma unroll
   for (int c = 0; c < kBlk; ++c) {
     float s = 0.0f;
@@ -316,6 +319,7 @@ __global__ __launch_bounds__(64 * kEncWaves, 3) void rabitq4_encode_kernel(const
     for (int j = 0; j < 8; ++j) {
       y[8 * c + j] = bf16r(y[8 * c + j] * kHadScale);
       s = __builtin_fmaf(y[8 * c + j], y[8 * c + j], s);
+      lowest = min(lowest, __float_as_int(y[8 * c + j]));
     }
     least = fminf(least, s);
     // the hardware root (within 1 unit of the last place) rounds to the same
@@ -332,6 +336,12 @@ __global__ __launch_bounds__(64 * kEncWaves, 3) void rabitq4_encode_kernel(const
       for (int j = 0; j < 8; ++j) s = s + y[8 * c + j] * y[8 * c + j];
       rad[c] = bf16r(__builtin_sqrtf(s));
     }
+  }
+  // a y that rounded to -0 (from under half of bf16's smallest value) becomes
+  // +0: from here on the sign bit of a y is y < 0
+  if (lowest == INT_MIN) {
+#pragma unroll
+    for (int d = 0; d < kDim; ++d) y[d] = y[d] + 0.0f;
   }
 
   // ---- blocks: direction, bucket, alpha, weight (PC:1170-1192) ----
