@@ -211,6 +211,30 @@ def test_decode_linear_units_and_k_ranges(M, K, N):
     assert torch.isfinite(normed[:, ~bad]).all() and not torch.isfinite(normed[:, bad]).any()
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (6, 3072, 4096), (5, 4096, 4096),                     # eight waves per unit, two chains each
+    (7, 2560, 8192), (13, 3328, 8200),                    # four waves; two long rows per wave, a last unit of 8 rows
+    (5, 3328, 17602), (9, 2688, 17602),                   # more units than the resident groups: two or three each
+    (16, 4352, 2890), (6, 9728, 1090), (5, 2560, 4896),   # LDS nearly full; rows past the first requests; a workgroup per tile
+])
+def test_decode_linear_normed_splits(M, K, N):
+    """The waves per unit, units per group and row lengths of the normed linear
+    at 5 rows and more, without and with silu * up, the latter over both halves
+    of the same weights.  Two bf16 units, as above."""
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    nw = (torch.rand(K, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
+    y = (ds.rms_norm(x, nw, 1e-6).float() @ w.float().T).to(torch.bfloat16)
+    out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    ds.decode_linear(x, w, out[:M], norm_w=nw, eps=1e-6)
+    _bf16_close(out[:M], y, ulps=2.0)
+    act = torch.full((M + 1, N // 2), 7.0, dtype=torch.bfloat16, device="cuda")
+    ds.decode_linear(x, w, act[:M], norm_w=nw, eps=1e-6, silu_mul=True)
+    _bf16_close(act[:M], torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:], ulps=2.0)
+    assert (out[M] == 7.0).all() and (act[M] == 7.0).all()
+
+
 def test_decode_linear_rejects_bad_shapes():
     from zoomkv_revision_amd._lib import ZkvError
     x = torch.zeros(4, 200, dtype=torch.bfloat16, device="cuda")

@@ -304,12 +304,14 @@ __global__ __launch_bounds__(1024) void decode_rows_kernel(const LinearParams p,
 
 // Stages the M x K input rows into LDS (row stride ld elements), RMS-normalised:
 // bf16(x * rsqrt(mean(x^2) + eps) * w).  Wave w of nw takes rows w, w + nw, ...;
-// lane l holds 16-byte chunks l, l + 64, ... of a row, summed in that order.  load(), called ahead of the kernel's weight loads,
-// requests the first kChunks chunks of kRows rows per wave: a request behind the
-// weights waits for them.  The caller synchronises after run().
-template <int kRows>
+// lane l holds 16-byte chunks l, l + 64, ... of a row, summed in that order.
+// load(), called ahead of the kernel's weight loads, requests the first kChunks
+// chunks (512 kChunks elements) of kRows rows per wave; what is left of a longer
+// row is requested behind the weights and waits for them, twice (decode_wide_kernel
+// with kChunks 5 and 8, 6144 x 4096, M = 6: 19.5 -> 17.6 us).  The caller
+// synchronises after run().
+template <int kRows, int kChunks>
 struct NormStage {
-  static constexpr int kChunks = 5;  // per lane: K <= 2560 needs no later load
   u32x4_t xv[kRows][kChunks], wv[kChunks];
 
   __device__ __forceinline__ void load_row(const LinearParams& p, int r, int m, int lane) {
@@ -320,7 +322,8 @@ struct NormStage {
   __device__ __forceinline__ void load(const LinearParams& p, int wave, int nw, int lane) {
     const int last = (p.K >> 3) - 1;
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) load_row(p, r, wave + r * nw, lane);
+    for (int r = 0; r < kRows; ++r)
+      if (r == 0 || wave + r * nw < p.M) load_row(p, r, wave + r * nw, lane);  // (uniform)
 #pragma unroll
     for (int j = 0; j < kChunks; ++j)
       wv[j] = reinterpret_cast<const u32x4_t*>(p.norm_w)[min(lane + 64 * j, last)];
@@ -385,19 +388,25 @@ struct NormStage {
 //
 // A workgroup of nw waves is nw / S groups; the S waves of a group share a
 // unit, wave `part` of it taking blocks part, part + S, ..., and group g of the
-// grid takes units g, g + (groups in the grid), ...  A block is four loads (4
-// KiB); each wave keeps four blocks in flight, across unit ends and from before
-// the x rows are staged.  The loads are the same on every path: one that some
+// grid takes units g, g + (groups in the grid), ... (one each for most of a
+// layer's projections, which have about as many units as groups fit the chip).
+// A block is four loads (4 KiB); each wave keeps four blocks in flight, across
+// unit ends and from before the x rows are staged.  The loads are the same on every path: one that some
 // path skips makes the compiler wait for the whole stream at each round (past
 // a wave's last block they re-read the start of an x row).
 //
 // The normalised x rows sit in LDS (16 bytes apart in their banks where there is
-// room).  Against a workgroup per unit, which stages the rows for every unit
-// and waits for them before its first weight load (us at M = 6 / 12 / 16):
-// qkv 13.5 / 15.6 / 20.3 -> 12.2 / 12.3 / 13.6, gate and up 31.1 / 50.5 / 84.3 ->
-// 22.1 / 23.7 / 24.5, head 195 / 312 / 587 -> 142 / 148 / 152.
+// room).  kLong: rows of more than 2560 elements, two rows of 4096 per wave
+// requested ahead of the weights instead of three of 2560 (249-254 VGPRs
+// instead of 204-209: a workgroup of eight waves per CU either way).  Against
+// a workgroup per unit, which stages the rows for every unit and waits for them
+// before its first weight load (us at M = 6 / 12 / 16): qkv 6144 x 2560 13.4 /
+// 15.4 / 19.8 -> 12.0 / 12.1 / 13.4, 6144 x 4096 19.2 / 27.9 / 29.4 -> 17.6 / 17.9 /
+// 19.6, gate and up 19456 x 2560 30.7 / 49.4 / 83.4 -> 22.0 / 23.7 / 24.4, 24576 x
+// 4096 51.6 / 103 / 112 -> 38.7 / 38.9 / 41.0, head 195 / 311 / 585 -> 142 / 149 /
+// 153.
 // ---------------------------------------------------------------------------
-template <int kEpi, int kA>
+template <int kEpi, int kA, bool kLong>
 __global__ __launch_bounds__(512) void decode_wide_kernel(const LinearParams p, int n_units, int S, int xs_ld) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int kDepth = 4;  // blocks in flight; a multiple of kA
@@ -424,7 +433,7 @@ __global__ __launch_bounds__(512) void decode_wide_kernel(const LinearParams p, 
     else
       return min(16 * u + r, N - 1);
   };
-  NormStage<3> stage;
+  NormStage<kLong ? 2 : 3, kLong ? 8 : 5> stage;
   stage.load(p, wave, nw, lane);
   float res0[4];  // the first unit's residual: lane (c, g) ends with rows 4g + i of x row c
   if constexpr (kEpi == kEpiResidual) {
@@ -639,7 +648,7 @@ __global__ __launch_bounds__(64 * kGemvWaves) void decode_stream_kernel(const Li
       return min(u * kR + r, N - 1);
     }
   };
-  NormStage<1> stage;
+  NormStage<1, 5> stage;
   if constexpr (kNorm) stage.load(p, wave, kGemvWaves, lane);
   // the first unit's residual (of the lane that stores it)
   const int o_idx = lane >> kShift, o_r = o_idx / kGemvMaxM, o_m = o_idx % kGemvMaxM;
@@ -879,11 +888,22 @@ extern "C" int zkv_decode_linear(const uint16_t* x, int64_t x_ld, int M, int K, 
   }
   if (norm_w && static_cast<int64_t>(n_tiles) * nkb >= 6144) {
     // 24 MB of weights and more: a workgroup per tile against this stream, M = 6,
-    // 4096 x 1024 (2048 blocks) 5.9 and 6.6 us, 6144 x 2560 (7680) 13.5 and 12.2.
-    // The chains of a unit's sum (nw of them) on at most four accumulators per
-    // wave and the rest as waves; eight waves (six where a unit takes one) stage
-    // the rows.
-    const int per_wave = std::min(nw, 4), S = nw / per_wave;
+    // 4096 x 1024 (2048 blocks) 5.9 and 6.6 us, 6144 x 2048 (6144) 11.7 and 10.3,
+    // 6144 x 2560 (7680) 13.4 and 12.0.
+    // The nw chains of a unit's sum are nw / S accumulators in each of S waves.  S
+    // is the split whose waves take the fewest rounds of kDepth blocks: 2048 waves
+    // run at a time, and a wave loads whole rounds.  Fewer waves per unit unless
+    // more save a sixteenth: 8192 x 2560, M = 6, S = 2 (128 workgroups) 16.3 us, S = 4
+    // (256) 12.8; 4096 x 4096 S = 4 17.0, S = 8 11.8; 24576 x 4096 S = 2 53, S = 4
+    // 38.7; the head of 4096, 151936 rows, S = 2 (160 rounds) 237, S = 4 (152) 242.
+    int S = 0, best = 0;
+    for (int t = std::max(nw / 4, 1); t <= std::min(nw, 8); t *= 2) {
+      const int turns = static_cast<int>((static_cast<int64_t>(n_tiles) * t + 2047) / 2048);
+      const int rounds = turns * (((nkb + t - 1) / t + 3) / 4);
+      if (S == 0 || 16 * rounds < 15 * best) best = rounds, S = t;
+    }
+    // eight waves (six where a unit takes one) stage the rows
+    const int per_wave = nw / S;
     int nwv = S == 1 ? 6 : 8;
     // (one unit's chains always fit: the requirement above)
     if (S > 1 && x_bytes + static_cast<size_t>(nwv) * per_wave * 1024 > 160 * 1024) nwv = S;
@@ -891,19 +911,29 @@ extern "C" int zkv_decode_linear(const uint16_t* x, int64_t x_ld, int M, int K, 
     // x rows 16 bytes apart in their banks where the LDS holds the padding
     const int xs_ld = x_bytes + M * 16 + red_bytes <= 160 * 1024 ? K + 8 : K;
     const size_t lds = static_cast<size_t>(M) * xs_ld * 2 + red_bytes;
-    // (a stream per wave from 2048 units on: one workgroup per CU, M = 16 head
-    // 152 us against 167 with a workgroup per six units)
-    const int grid = std::min((n_tiles + nwv / S - 1) / (nwv / S), n_tiles >= 2048 ? 256 : 1 << 30);
-#define ZKV_WIDE(E)                                                                               \
-  do {                                                                                            \
-    if (per_wave == 4) ZKV_LAUNCH(decode_wide_kernel<E ZKV_COMMA 4>, grid, 64 * nwv, lds, p, n_tiles, S, xs_ld); \
-    else if (per_wave == 2) ZKV_LAUNCH(decode_wide_kernel<E ZKV_COMMA 2>, grid, 64 * nwv, lds, p, n_tiles, S, xs_ld); \
-    else ZKV_LAUNCH(decode_wide_kernel<E ZKV_COMMA 1>, grid, 64 * nwv, lds, p, n_tiles, S, xs_ld); \
+    // a workgroup per CU, what the registers allow: one that waits for another's
+    // end would stage the rows again
+    const int grid = std::min((n_tiles + nwv / S - 1) / (nwv / S), 256);
+    const bool long_rows = K > 2560;
+#define ZKV_WIDE_L(E, A, L) \
+  ZKV_LAUNCH(decode_wide_kernel<E ZKV_COMMA A ZKV_COMMA L>, grid, 64 * nwv, lds, p, n_tiles, S, xs_ld)
+#define ZKV_WIDE_A(E, A)                        \
+  do {                                          \
+    if (long_rows) ZKV_WIDE_L(E, A, true);      \
+    else ZKV_WIDE_L(E, A, false);               \
+  } while (0)
+#define ZKV_WIDE(E)                             \
+  do {                                          \
+    if (per_wave == 4) ZKV_WIDE_A(E, 4);        \
+    else if (per_wave == 2) ZKV_WIDE_A(E, 2);   \
+    else ZKV_WIDE_A(E, 1);                      \
   } while (0)
     if (epilogue == kEpiNone) ZKV_WIDE(kEpiNone);
     else if (epilogue == kEpiResidual) ZKV_WIDE(kEpiResidual);
     else ZKV_WIDE(kEpiSiluMul);
 #undef ZKV_WIDE
+#undef ZKV_WIDE_A
+#undef ZKV_WIDE_L
     return check_launch("decode_wide_kernel");
   }
   if (!norm_w) {
