@@ -235,6 +235,32 @@ def test_decode_linear_normed_splits(M, K, N):
     assert (out[M] == 7.0).all() and (act[M] == 7.0).all()
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (1, 512, 12288), (2, 512, 12289), (3, 384, 5),        # a lane per 16 bytes of a row: one unit per wave, some two, a lone one
+    (4, 2048, 3072), (1, 2048, 3073), (2, 1664, 2050),    # split K, one chunk per wave: 768 units, 769, a short last chunk
+    (4, 2176, 2050),                                      # a wave with two chunks
+])
+def test_decode_linear_stream_units(M, K, N):
+    """Where the waves of the stream kernel (4 rows and fewer, no norm) have
+    one item or more, plain, with the residual and as silu * up."""
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    res = torch.randn(M, N, generator=g, device="cuda").to(torch.bfloat16)
+    y = (x.float() @ w.float().T).to(torch.bfloat16)
+    out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    ds.decode_linear(x, w, out[:M])
+    _bf16_close(out[:M], y)
+    ds.decode_linear(x, w, out[:M], residual=res)
+    _bf16_close(out[:M], res + y, ulps=2.0)
+    assert (out[M] == 7.0).all()
+    if N % 2 == 0:
+        act = torch.full((M + 1, N // 2), 7.0, dtype=torch.bfloat16, device="cuda")
+        ds.decode_linear(x, w, act[:M], silu_mul=True)
+        _bf16_close(act[:M], torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:], ulps=2.0)
+        assert (act[M] == 7.0).all()
+
+
 def test_decode_linear_rejects_bad_shapes():
     from zoomkv_revision_amd._lib import ZkvError
     x = torch.zeros(4, 200, dtype=torch.bfloat16, device="cuda")

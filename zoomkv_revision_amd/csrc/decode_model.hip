@@ -620,10 +620,12 @@ __device__ __forceinline__ u32x4_t stream_load(const uint16_t* base, int off) {
 // launcher uses it for K >= 4 chunks), and the waves' partial sums meet in
 // LDS at the unit's end; the workgroups take units blockIdx.x, blockIdx.x +
 // gridDim.x, ...
-template <int kEpi, bool kNorm, bool kSplit>
+// kD: items in flight; 1 where no wave has a second item (2048 x 2048, M = 1,
+// two loads of which the second only re-reads x: 4.8 us, one: 4.0).
+template <int kEpi, bool kNorm, bool kSplit, int kD>
 __global__ __launch_bounds__(64 * kGemvWaves) void decode_stream_kernel(const LinearParams p, int n_units) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  constexpr int kR = kGemvRows, kD = 2;  // rows per unit, items in flight
+  constexpr int kR = kGemvRows;
   constexpr int kV = kR * kGemvMaxM;     // values per lane: acc[r * 4 + m]
   constexpr int kShift = 2;              // lanes 4 i .. 4 i + 3 end with value i
   float* red = reinterpret_cast<float*>(lds);  // kSplit: [waves][64] partial sums
@@ -869,21 +871,26 @@ extern "C" int zkv_decode_linear(const uint16_t* x, int64_t x_ld, int M, int K, 
     const bool split = rows < 8192 && n_chunks >= kGemvWaves && !norm_w;
     const int per_unit = epilogue == kEpiSiluMul ? kGemvRows / 2 : kGemvRows;
     const int n_units = (rows + per_unit - 1) / per_unit;
-    const int grid = std::max(1, std::min(split ? n_units : (n_units + kGemvWaves - 1) / kGemvWaves, 768));
+    const int n_groups = split ? n_units : (n_units + kGemvWaves - 1) / kGemvWaves;
+    const int grid = std::max(1, std::min(n_groups, 768));
+    // one unit and one chunk of it for each wave (a norm's staging hides the rest)
+    const bool once = !norm_w && n_groups <= 768 && n_chunks == (split ? kGemvWaves : 1);
     const size_t lds = (split ? kGemvWaves * 64 * 4 : 0) + (norm_w ? x_bytes : 0);
-#define ZKV_GEMV(E)                                                                                   \
-  do {                                                                                                \
-    if (norm_w)                                                                                       \
-      ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA true ZKV_COMMA false>, grid, 64 * kGemvWaves, lds, p, n_units); \
-    else if (split)                                                                                   \
-      ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA false ZKV_COMMA true>, grid, 64 * kGemvWaves, lds, p, n_units); \
-    else                                                                                              \
-      ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA false ZKV_COMMA false>, grid, 64 * kGemvWaves, lds, p, n_units); \
+#define ZKV_GEMV_L(E, NORM, SPLIT, D)                                                                    \
+  ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA NORM ZKV_COMMA SPLIT ZKV_COMMA D>, grid, 64 * kGemvWaves, lds, p, n_units)
+#define ZKV_GEMV(E)                                       \
+  do {                                                    \
+    if (norm_w) ZKV_GEMV_L(E, true, false, 2);            \
+    else if (split && once) ZKV_GEMV_L(E, false, true, 1); \
+    else if (split) ZKV_GEMV_L(E, false, true, 2);        \
+    else if (once) ZKV_GEMV_L(E, false, false, 1);        \
+    else ZKV_GEMV_L(E, false, false, 2);                  \
   } while (0)
     if (epilogue == kEpiNone) ZKV_GEMV(kEpiNone);
     else if (epilogue == kEpiResidual) ZKV_GEMV(kEpiResidual);
     else ZKV_GEMV(kEpiSiluMul);
 #undef ZKV_GEMV
+#undef ZKV_GEMV_L
     return check_launch("decode_stream_kernel");
   }
   if (norm_w && static_cast<int64_t>(n_tiles) * nkb >= 6144) {
