@@ -239,10 +239,11 @@ def test_decode_linear_normed_splits(M, K, N):
     (1, 512, 12288), (2, 512, 12289), (3, 384, 5),        # a lane per 16 bytes of a row: one unit per wave, some two, a lone one
     (4, 2048, 3072), (1, 2048, 3073), (2, 1664, 2050),    # split K, one chunk per wave: 768 units, 769, a short last chunk
     (4, 2176, 2050),                                      # a wave with two chunks
+    (3, 1152, 40002), (4, 1152, 39998), (2, 4096, 40000),  # units of 8 rows, the last of 2 (silu * up: of 1); of 4; of 4 (8)
 ])
 def test_decode_linear_stream_units(M, K, N):
     """Where the waves of the stream kernel (4 rows and fewer, no norm) have
-    one item or more, plain, with the residual and as silu * up."""
+    one item or more and where its units change, plain, with the residual and as silu * up."""
     g = torch.Generator(device="cuda").manual_seed(M + K + N)
     x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
     w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16)

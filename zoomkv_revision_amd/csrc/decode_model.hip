@@ -538,10 +538,10 @@ __global__ __launch_bounds__(512) void decode_wide_kernel(const LinearParams p, 
 
 // ---------------------------------------------------------------------------
 // The same linear for M <= 4 input rows as a weight stream.  A unit of work
-// is 4 weight rows over all of K (silu * up: 2 gate rows and the matching up
-// rows); every wave takes units gw, gw + (waves in the grid), ... and walks
+// is kR = 4 (or 8) weight rows over all of K (silu * up: kR / 2 gate rows and the
+// matching up rows); every wave takes units gw, gw + (waves in the grid), ... and walks
 // their (unit, 512-element chunk) items with two items in flight: each item is
-// 4 loads of 1 KiB of one weight row (64 lanes x 16 B, whole cache lines,
+// kR loads of 1 KiB of one weight row (64 lanes x 16 B, whole cache lines,
 // nontemporal) and, without a norm, the x rows' 16 B.  The loads are the same
 // on every path, as in decode_wide_kernel.  With the norm, the workgroup stages
 // the normalised x rows in LDS once (the grid is at most a few workgroups per
@@ -549,7 +549,7 @@ __global__ __launch_bounds__(512) void decode_wide_kernel(const LinearParams p, 
 // ahead of the first weights.  v_dot2_f32_bf16 accumulates w x x in fp32; at
 // the unit's last chunk the lanes' partial sums are reduce-scattered with
 // shuffles and the epilogue (that of decode_linear_kernel) runs by lane
-// quadruples.  Waves never wait for each other after the staging.
+// quadruples (kR = 8: pairs).  Waves never wait for each other after the staging.
 //
 // Bound: HBM, behind ~3 us of launch, first latency and last sums.  Qwen3-4B
 // projections at M = 4, cold weights, us: a plain read of the weights / with
@@ -561,7 +561,6 @@ __global__ __launch_bounds__(512) void decode_wide_kernel(const LinearParams p, 
 constexpr int kGemvMaxM = 4;
 constexpr int kGemvChunk = 512;  // elements of one row read by one wave instruction
 constexpr int kGemvWaves = 4;
-constexpr int kGemvRows = 4;     // weight rows per unit
 
 typedef __bf16 bf16x2v_t __attribute__((ext_vector_type(2)));
 
@@ -593,15 +592,28 @@ __device__ __forceinline__ void rs_step(const float (&v)[N], float (&o)[N / 2], 
   }
 }
 
-// The sum over the 64 lanes of value lane / 4 of the 16 per-lane values.
-__device__ __forceinline__ float lane_reduce(const float (&acc)[16], int lane) {
-  float a[8], b[4], c[2], d[1];
-  rs_step<16>(acc, a, lane, 32);
-  rs_step<8>(a, b, lane, 16);
-  rs_step<4>(b, c, lane, 8);
-  rs_step<2>(c, d, lane, 4);
-  float s = d[0] + __shfl_xor(d[0], 2);
-  return s + __shfl_xor(s, 1);
+// The sum over the 64 lanes of value lane * kV / 64 of the kV per-lane values
+// (the same additions for any kV).
+template <int kV>
+__device__ __forceinline__ float lane_reduce(const float (&acc)[kV], int lane) {
+  static_assert(kV == 16 || kV == 32, "4 or 8 rows of 4");
+  if constexpr (kV == 32) {
+    float a[16], b[8], c[4], d[2], e[1];
+    rs_step<32>(acc, a, lane, 32);
+    rs_step<16>(a, b, lane, 16);
+    rs_step<8>(b, c, lane, 8);
+    rs_step<4>(c, d, lane, 4);
+    rs_step<2>(d, e, lane, 2);
+    return e[0] + __shfl_xor(e[0], 1);
+  } else {
+    float a[8], b[4], c[2], d[1];
+    rs_step<16>(acc, a, lane, 32);
+    rs_step<8>(a, b, lane, 16);
+    rs_step<4>(b, c, lane, 8);
+    rs_step<2>(c, d, lane, 4);
+    const float s = d[0] + __shfl_xor(d[0], 2);
+    return s + __shfl_xor(s, 1);
+  }
 }
 
 // 16 bytes of global memory at a wave-uniform base plus a lane's element
@@ -621,13 +633,12 @@ __device__ __forceinline__ u32x4_t stream_load(const uint16_t* base, int off) {
 // LDS at the unit's end; the workgroups take units blockIdx.x, blockIdx.x +
 // gridDim.x, ...
 // kD: items in flight; 1 where no wave has a second item (2048 x 2048, M = 1,
-// two loads of which the second only re-reads x: 4.8 us, one: 4.0).
-template <int kEpi, bool kNorm, bool kSplit, int kD>
+// two loads of which the second only re-reads x: 4.8 us, one: 4.15).
+template <int kEpi, bool kNorm, bool kSplit, int kR, int kD>
 __global__ __launch_bounds__(64 * kGemvWaves) void decode_stream_kernel(const LinearParams p, int n_units) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  constexpr int kR = kGemvRows;
-  constexpr int kV = kR * kGemvMaxM;     // values per lane: acc[r * 4 + m]
-  constexpr int kShift = 2;              // lanes 4 i .. 4 i + 3 end with value i
+  constexpr int kV = kR * kGemvMaxM;       // values per lane: acc[r * 4 + m]
+  constexpr int kShift = kR == 8 ? 1 : 2;  // value i ends in lanes i << kShift on
   float* red = reinterpret_cast<float*>(lds);  // kSplit: [waves][64] partial sums
   uint16_t* xs = reinterpret_cast<uint16_t*>(lds + (kSplit ? kGemvWaves * 64 * 4 : 0));  // normalised x [M][K]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -869,22 +880,35 @@ extern "C" int zkv_decode_linear(const uint16_t* x, int64_t x_ld, int M, int K, 
     const int rows = epilogue == kEpiSiluMul ? N / 2 : N;
     const int n_chunks = (K + kGemvChunk - 1) / kGemvChunk;
     const bool split = rows < 8192 && n_chunks >= kGemvWaves && !norm_w;
-    const int per_unit = epilogue == kEpiSiluMul ? kGemvRows / 2 : kGemvRows;
+    // without a norm each item loads the x rows too: units of 8 rows halve that
+    // from 40000 weight rows on; 151936 x 2560, M = 1 / 4, us: 4 rows 113 / 124, 8 rows
+    // 112 / 113; 65536 x 2048 50.1 / 51.3 and 46.4 / 47.0.  Fewer rows give the waves
+    // too few units (36000 x 2048 24.6 / 25.2 and 27.2 / 27.3), one x row and rows of
+    // 1024 have little to halve (65536 x 6144 119 and 122 at M = 1; 151936 x 1024 47.4
+    // / 48.0 and 48.8 / 48.5), and 8 rows whole multiples of 8 KiB apart meet on the
+    // same channels (65536 x 4096 84 / 87 and 110 / 113; silu * up, whose rows are two
+    // runs of 4, not: 40000 x 4096 57.7 / 59.8 and 53.4 / 53.4).
+    const bool tall = !norm_w && N >= 40000 && K > 1024 && (M >= 2 || K < 4096) &&
+                      (K % 4096 != 0 || epilogue == kEpiSiluMul);
+    const int R = tall ? 8 : 4;
+    const int per_unit = epilogue == kEpiSiluMul ? R / 2 : R;
     const int n_units = (rows + per_unit - 1) / per_unit;
     const int n_groups = split ? n_units : (n_units + kGemvWaves - 1) / kGemvWaves;
     const int grid = std::max(1, std::min(n_groups, 768));
     // one unit and one chunk of it for each wave (a norm's staging hides the rest)
     const bool once = !norm_w && n_groups <= 768 && n_chunks == (split ? kGemvWaves : 1);
     const size_t lds = (split ? kGemvWaves * 64 * 4 : 0) + (norm_w ? x_bytes : 0);
-#define ZKV_GEMV_L(E, NORM, SPLIT, D)                                                                    \
-  ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA NORM ZKV_COMMA SPLIT ZKV_COMMA D>, grid, 64 * kGemvWaves, lds, p, n_units)
-#define ZKV_GEMV(E)                                       \
-  do {                                                    \
-    if (norm_w) ZKV_GEMV_L(E, true, false, 2);            \
-    else if (split && once) ZKV_GEMV_L(E, false, true, 1); \
-    else if (split) ZKV_GEMV_L(E, false, true, 2);        \
-    else if (once) ZKV_GEMV_L(E, false, false, 1);        \
-    else ZKV_GEMV_L(E, false, false, 2);                  \
+#define ZKV_GEMV_L(E, NORM, SPLIT, R, D)                                                                 \
+  ZKV_LAUNCH(decode_stream_kernel<E ZKV_COMMA NORM ZKV_COMMA SPLIT ZKV_COMMA R ZKV_COMMA D>, grid, 64 * kGemvWaves, lds, \
+             p, n_units)
+#define ZKV_GEMV(E)                                          \
+  do {                                                       \
+    if (norm_w) ZKV_GEMV_L(E, true, false, 4, 2);            \
+    else if (tall) ZKV_GEMV_L(E, false, false, 8, 2);        \
+    else if (split && once) ZKV_GEMV_L(E, false, true, 4, 1); \
+    else if (split) ZKV_GEMV_L(E, false, true, 4, 2);        \
+    else if (once) ZKV_GEMV_L(E, false, false, 4, 1);        \
+    else ZKV_GEMV_L(E, false, false, 4, 2);                  \
   } while (0)
     if (epilogue == kEpiNone) ZKV_GEMV(kEpiNone);
     else if (epilogue == kEpiResidual) ZKV_GEMV(kEpiResidual);
