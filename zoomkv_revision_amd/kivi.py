@@ -80,25 +80,28 @@ def cache_prefill(keys: torch.Tensor, values: torch.Tensor, sink: int, local: in
     complete chunks are encoded at chunk 0 as ``chunk_encode`` does (the metadata
     tensors are its).  Returns the number of chunks.  Everything is bf16 and
     16-byte aligned (``cache_prefill_takes``)."""
-    require_gpu(keys, values, k_rows, v_rows, chunk_min, chunk_max, chunk_centroid, chunk_valid, packed_K)
     bs, kv, n, _ = keys.shape
+    n_max = chunk_min.shape[2]
+    # the extents the kernel writes are k_rows' rows and chunk_min's chunks
+    for name, t in (("k_rows", k_rows), ("v_rows", v_rows)):
+        _check_bf16(name, t)
+        if tuple(t.shape) != (bs, kv, k_rows.shape[2], HEAD_DIM) or t.stride(3) != 1 or t.stride(2) != HEAD_DIM \
+                or t.stride() != k_rows.stride():
+            raise ValueError(f"{name} must be [{bs}, {kv}, rows, {HEAD_DIM}] with contiguous rows, as k_rows; "
+                             f"got {tuple(t.shape)} stride {t.stride()}")
+    for name, t, dtype, tail in (("chunk_min", chunk_min, torch.bfloat16, (HEAD_DIM,)),
+                                 ("chunk_max", chunk_max, torch.bfloat16, (HEAD_DIM,)),
+                                 ("chunk_centroid", chunk_centroid, torch.bfloat16, (HEAD_DIM,)),
+                                 ("chunk_valid", chunk_valid, torch.bool, ()),
+                                 ("packed_K", packed_K, torch.int32, (16, chunk_size))):
+        if t.dtype != dtype:
+            raise TypeError(f"{name} must be {dtype}; got {t.dtype}")
+        if tuple(t.shape) != (bs, kv, n_max, *tail) or not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous {[bs, kv, n_max, *tail]}; got {tuple(t.shape)}")
+    require_gpu(keys, values, k_rows, v_rows, chunk_min, chunk_max, chunk_centroid, chunk_valid, packed_K)
     ret = n - sink - local
     if keys.shape != values.shape or ret < 0 or not cache_prefill_takes(keys, values):
         raise ValueError("cache_prefill: bf16 keys / values of one shape with 16-byte aligned rows")
-    for name, t in (("k_rows", k_rows), ("v_rows", v_rows)):
-        _check_bf16(name, t)
-        if tuple(t.shape[:2]) != (bs, kv) or t.stride(3) != 1 or t.stride(2) != HEAD_DIM or t.stride() != k_rows.stride():
-            raise ValueError(f"{name} must be [bs, kv, rows, 128] with contiguous rows")
-    for name, t in (("chunk_min", chunk_min), ("chunk_max", chunk_max), ("chunk_centroid", chunk_centroid)):
-        _check_bf16(name, t)
-        if not t.is_contiguous():
-            raise ValueError(f"{name} must be contiguous")
-    if chunk_valid.dtype != torch.bool or packed_K.dtype != torch.int32:
-        raise TypeError("chunk_valid must be bool and packed_K int32")
-    n_max = chunk_min.shape[2]
-    if tuple(packed_K.shape) != (bs, kv, n_max, 16, chunk_size) or not packed_K.is_contiguous():
-        raise ValueError(f"packed_K must be contiguous [{bs}, {kv}, {n_max}, 16, {chunk_size}]; "
-                         f"got {tuple(packed_K.shape)}")
     ks, vs, rs = keys.stride(), values.stride(), k_rows.stride()
     check(lib().zkv_cache_prefill(
         ptr(keys), ks[0], ks[1], ks[2], ptr(values), vs[0], vs[1], vs[2], bs, kv, sink, ret, local,
