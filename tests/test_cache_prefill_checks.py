@@ -49,3 +49,26 @@ def test_matching_buffers_pass_the_host_checks():
     """... up to the one that they are on the GPU."""
     with pytest.raises(ZkvError, match="device tensors"):
         kivi.cache_prefill(**_args())
+
+
+class _Rows:
+    """A [2, 3, 80, 128] tensor's layout on some device."""
+    dtype, is_cuda, shape = torch.bfloat16, True, (2, 3, 80, 128)
+
+    def __init__(self, index, ptr=4096):
+        self.device, self._ptr = torch.device("cuda", index), ptr
+
+    def stride(self, dim=None):
+        s = (80 * 3 * 128, 128, 3 * 128, 1)
+        return s if dim is None else s[dim]
+
+    def data_ptr(self):
+        return self._ptr
+
+
+def test_rows_of_two_devices_are_not_taken_in_place():
+    """polar_cache copies such a prompt piece by piece: a kernel of one device
+    cannot read the other's memory."""
+    assert kivi.cache_prefill_takes(_Rows(0), _Rows(0))
+    assert not kivi.cache_prefill_takes(_Rows(0), _Rows(0, ptr=4098))
+    assert not kivi.cache_prefill_takes(_Rows(0), _Rows(1))

@@ -99,6 +99,8 @@ def cache_prefill(keys: torch.Tensor, values: torch.Tensor, sink: int, local: in
         if tuple(t.shape) != (bs, kv, n_max, *tail) or not t.is_contiguous():
             raise ValueError(f"{name} must be contiguous {[bs, kv, n_max, *tail]}; got {tuple(t.shape)}")
     require_gpu(keys, values, k_rows, v_rows, chunk_min, chunk_max, chunk_centroid, chunk_valid, packed_K)
+    if any(t.device != keys.device for t in (k_rows, v_rows, chunk_min, chunk_max, chunk_centroid, chunk_valid, packed_K)):
+        raise ValueError("cache_prefill: all tensors on one device")
     ret = n - sink - local
     if keys.shape != values.shape or ret < 0 or not cache_prefill_takes(keys, values):
         raise ValueError("cache_prefill: bf16 keys / values of one shape with 16-byte aligned rows")
@@ -112,8 +114,9 @@ def cache_prefill(keys: torch.Tensor, values: torch.Tensor, sink: int, local: in
 
 def cache_prefill_takes(*rows: torch.Tensor) -> bool:
     """Whether ``cache_prefill`` reads these [bs, kv, n, 128] tensors in place."""
-    return all(t.dtype == torch.bfloat16 and t.is_cuda and t.shape[-1] == HEAD_DIM and t.stride(-1) == 1
-               and not any(s % 8 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0 and t.shape[2] < 2 ** 20
+    return all(t.dtype == torch.bfloat16 and t.is_cuda and t.device == rows[0].device
+               and t.shape[-1] == HEAD_DIM and t.stride(-1) == 1 and not any(s % 8 for s in t.stride()[:3])
+               and t.data_ptr() % 16 == 0 and t.shape[2] < 2 ** 20
                for t in rows)
 
 
