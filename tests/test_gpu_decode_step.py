@@ -262,6 +262,27 @@ def test_decode_linear_stream_units(M, K, N):
         assert (act[M] == 7.0).all()
 
 
+@pytest.mark.parametrize("K,N", [(512, 1030), (2560, 4896), (2560, 6144), (3328, 17602), (4352, 2890), (256, 98304)])
+@pytest.mark.parametrize("M", [2, 6, 16])
+def test_decode_linear_norm_with_residual(M, K, N):
+    """Norm and residual in one call, under and over 6144 blocks of 4 KiB, with
+    one unit and with several per group of waves, out of place and in place.
+    Two bf16 units, as above."""
+    if M * K * 2 + 16384 > 160 * 1024:
+        pytest.skip("x rows past the LDS")
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    nw = (torch.rand(K, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
+    res = 4 * torch.randn(M, N, generator=g, device="cuda").to(torch.bfloat16)
+    ref = res + (ds.rms_norm(x, nw, 1e-6).float() @ w.float().T).to(torch.bfloat16)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    ds.decode_linear(x, w, out, norm_w=nw, eps=1e-6, residual=res)
+    _bf16_close(out, ref, ulps=2.0)
+    ds.decode_linear(x, w, res, norm_w=nw, eps=1e-6, residual=res)
+    assert torch.equal(res, out)
+
+
 def test_decode_linear_rejects_bad_shapes():
     from zoomkv_revision_amd._lib import ZkvError
     x = torch.zeros(4, 200, dtype=torch.bfloat16, device="cuda")
