@@ -208,11 +208,14 @@ def test_prefill_launch_writes_what_the_separate_steps_write(monkeypatch, chunk,
         cache.valid_start = [valid_start] * 2
         for t in (cache.unified_keys[0], cache.unified_values[0], cache._chunk_carry_keys[0]):
             t.fill_(7.0)
+        calls, launch = [], kivi.cache_prefill
+        monkeypatch.setattr(kivi, "cache_prefill", lambda *a: calls.append(a) or launch(*a))
         if not one_launch:
             monkeypatch.setattr(kivi, "cache_prefill_takes", lambda *t: False)
         for b in range(0, 2, rows):
             cache.prefill_update_kv_cache(None, k[b:b + rows], v[b:b + rows], 0, b)
         monkeypatch.undo()
+        assert len(calls) == (2 // rows if one_launch else 0)
         state = (cache.current_seq_len, cache.cpu_valid_end, cache._chunk_valid_end, cache._chunk_carry_count,
                  cache.context)
         return state, [cache.unified_keys[0], cache.unified_values[0], cache._chunk_key_min_gpu[0],
