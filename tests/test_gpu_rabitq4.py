@@ -118,13 +118,13 @@ def _edge_keys(g, n):
 
 
 @pytest.mark.parametrize("bs,kv,n,t0,thresholds", [
-    (1, 1, 41024, 0, None),                      # whole tiles
-    (1, 5, 8261, 3, None),                       # a last tile of 5 keys, odd first token
-    (2, 3, 7039, 1, "small"),                    # a threshold below the table: the general path in the tiles' launch
-    (1, 8, 5184, 0, "unsorted"),                 # counts of unsorted, negative and equal levels
+    (1, 1, 49216, 0, None),                      # whole tiles
+    (1, 5, 9861, 3, None),                       # a last tile of 5 keys, odd first token
+    (2, 3, 8255, 1, "small"),                    # a threshold below the table: the general path in the tiles' launch
+    (1, 8, 6208, 0, "unsorted"),                 # counts of unsorted, negative and equal levels
 ])
 def test_encode_tiles_match_short_calls(bs, kv, n, t0, thresholds):
-    """Calls of 40960 keys and more (a lane per key) write the bits of calls of
+    """Calls of 49152 keys and more (a lane per key) write the bits of calls of
     a few keys (16 lanes per key, checked against the oracle above), special
     rows included; NaN weights are NaN in both."""
     zk = _zk()
@@ -140,7 +140,7 @@ def test_encode_tiles_match_short_calls(bs, kv, n, t0, thresholds):
                   torch.full((bs, kv, 16, t0 + n + 2), 7.0, dtype=torch.bfloat16, device="cuda"),
                   torch.full((bs, kv, 16, t0 + n + 2, 4), 0xCD, dtype=torch.uint8, device="cuda"))
     got, want = mk(), mk()
-    assert bs * kv * n >= 40960
+    assert bs * kv * n >= 49152
     zk.encode_into(keys, signs, thr, ctr, *got, t0)
     for i in range(0, n, 2000):
         zk.encode_into(keys[:, :, i:i + 2000], signs, thr, ctr, *want, t0 + i)
@@ -154,9 +154,9 @@ def test_encode_tiles_match_short_calls(bs, kv, n, t0, thresholds):
 def test_encode_tiles_round_to_minus_zero(rng):
     """y rounds to -0 where a bf16-subnormal quotient is what two cancelling
     entries leave: a -0 is not below zero, so its sign bit is 1 (y >= 0), in a
-    call of 40960 keys as in one of a few."""
+    call of 49152 keys as in one of a few."""
     zk = _zk()
-    n, special = 40964, 70
+    n, special = 49156, 70
     sg = np.where(rng.integers(0, 2, 128) == 1, 1.0, -1.0).astype(np.float32)
     x = rng.standard_normal((n, 128)).astype(np.float32)
     x[:special:3] = 0.0

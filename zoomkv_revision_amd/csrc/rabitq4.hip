@@ -672,9 +672,10 @@ extern "C" int zkv_rabitq4_encode(const uint16_t* keys, int64_t k_sb, int64_t k_
   const int64_t n_tiles = static_cast<int64_t>(bs) * kv * tiles_per_bh;
   // A tile takes its wave ~11 us whatever it holds, and 3072 run at a time; 16
   // lanes per key take ~0.25 us per 1000 keys over the whole chip.  8 heads of
-  // 1 / 4096 / 6144 / 16384 keys: 18.6 / 13.5 / 14.3 / 22.6 us by tiles, 3.5 /
-  // 11.2 / 18.1 / 41.8 us on 16 lanes (the last two with IEEE divisions).
-  if (p.rows >= 40960 && p.rows >= 48 * n_tiles) {
+  // 4096 / 5120 / 6144 / 8192 / 16384 keys: 13.5 / 14.0 / 14.5 / 15.3 / 22.6 us by
+  // tiles, 11.1 / 12.7 / 14.3 / 18.2 / 32.3 us on 16 lanes; 4096 heads of 16 / 33 / 49
+  // keys, a tile each: 31.5 / 34.4 / 36.8 and 17.6 / 33.9 / 48.7 us.
+  if (p.rows >= 49152 && p.rows >= 48 * n_tiles) {
     rabitq4_encode_kernel<<<static_cast<unsigned>((n_tiles + kEncWaves - 1) / kEncWaves), 64 * kEncWaves, 0, s>>>(
         p, tiles_per_bh, n_tiles);
     return check_launch("rabitq4_encode_kernel");
