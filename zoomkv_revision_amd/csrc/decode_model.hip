@@ -401,10 +401,11 @@ struct NormStage {
 // instead of 204-209: a workgroup of eight waves per CU either way).  Against
 // a workgroup per unit, which stages the rows for every unit and waits for them
 // before its first weight load (us at M = 6 / 12 / 16): qkv 6144 x 2560 13.4 /
-// 15.4 / 19.8 -> 12.0 / 12.1 / 13.4, 6144 x 4096 19.2 / 27.9 / 29.4 -> 17.6 / 17.9 /
-// 19.6, gate and up 19456 x 2560 30.7 / 49.4 / 83.4 -> 22.0 / 23.7 / 24.4, 24576 x
-// 4096 51.6 / 103 / 112 -> 38.7 / 38.9 / 41.0, head 195 / 311 / 585 -> 142 / 149 /
-// 153.
+// 15.4 / 19.8 -> 11.3 / 11.5 / 13.0, 6144 x 4096 19.3 / 26.9 / 29.3 -> 17.1 / 17.5 /
+// 19.6, gate and up 19456 x 2560 30.9 / 49.5 / 83.8 -> 21.5 / 23.4 / 24.2, 24576 x
+// 4096 51.4 / 103 / 111 -> 38.4 / 38.7 / 40.9, head 196 / 312 / 583 -> 142 / 148 /
+// 152.  (Slower by 2-3% at M = 5 only, of what was measured: 8192 x 4096 20.2 ->
+// 20.6, 9000 x 1536 10.8 -> 11.1.)
 // ---------------------------------------------------------------------------
 template <int kEpi, int kA, bool kLong>
 __global__ __launch_bounds__(512) void decode_wide_kernel(const LinearParams p, int n_units, int S, int xs_ld) {
@@ -919,14 +920,15 @@ extern "C" int zkv_decode_linear(const uint16_t* x, int64_t x_ld, int M, int K, 
   }
   if (norm_w && static_cast<int64_t>(n_tiles) * nkb >= 6144) {
     // 24 MB of weights and more: a workgroup per tile against this stream, M = 6,
-    // 4096 x 1024 (2048 blocks) 5.9 and 6.6 us, 6144 x 2048 (6144) 11.7 and 10.3,
-    // 6144 x 2560 (7680) 13.4 and 12.0.
+    // 4096 x 1024 (2048 blocks) 5.9 and 6.6 us, 6144 x 2048 (6144) 11.6 and 9.2,
+    // 6144 x 2560 (7680) 13.4 and 11.3.
     // The nw chains of a unit's sum are nw / S accumulators in each of S waves.  S
     // is the split whose waves take the fewest rounds of kDepth blocks: 2048 waves
     // run at a time, and a wave loads whole rounds.  Fewer waves per unit unless
     // more save a sixteenth: 8192 x 2560, M = 6, S = 2 (128 workgroups) 16.3 us, S = 4
-    // (256) 12.8; 4096 x 4096 S = 4 17.0, S = 8 11.8; 24576 x 4096 S = 2 53, S = 4
+    // (256) 12.8; 4096 x 4096 S = 4 17.0, S = 8 11.8; 24576 x 4096 S = 2 54, S = 4
     // 38.7; the head of 4096, 151936 rows, S = 2 (160 rounds) 237, S = 4 (152) 242.
+    // (The first figure of each with the long rows requested late.)
     int S = 0, best = 0;
     for (int t = std::max(nw / 4, 1); t <= std::min(nw, 8); t *= 2) {
       const int turns = static_cast<int>((static_cast<int64_t>(n_tiles) * t + 2047) / 2048);

@@ -102,7 +102,8 @@ __global__ __launch_bounds__(64, 3) void rabitq_encode_kernel(
       y[d + 1] = __builtin_fmaf(-b, signs[d + 1], t);
     }
     // (each sum is pinned where it is formed: sunk to its use below, it would
-    // keep all the row's words, or all of y, in registers and spill)
+    // keep all the row's words, or all of y, in registers and spill; so one of the
+    // 168 registers of three waves per SIMD does)
     asm volatile("" : "+v"(nsq));
   }
 #pragma unroll

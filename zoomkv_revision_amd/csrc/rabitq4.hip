@@ -186,8 +186,9 @@ constexpr int kEncWaves = 4;
 //  * the bucket and its center are one table read instead of 14 compares and
 //    selects; sign bits and codes enter their words by align instructions.
 // Half rows at a time (8 KiB of LDS per wave) let three waves share a SIMD:
-// 134 us with whole rows and two.  8 x 131072 keys: 123 us (3.1 TB/s, VALU
-// ~85% busy) against 292 us on 16 lanes per key.
+// 134 us with whole rows and two.  (Two of the 168 registers that leaves spill.)
+// 8 x 131072 keys: 125 us (3.1 TB/s, VALU ~85% busy; 124 without the look for a
+// -0) against 292 us on 16 lanes per key.
 __global__ __launch_bounds__(64 * kEncWaves, 3) void rabitq4_encode_kernel(const EncodeParams p, int tiles_per_bh,
                                                                           int64_t n_tiles) {
   // the table first: its reads then take their LDS offset as an immediate
