@@ -81,43 +81,49 @@ def cache_prefill(keys: torch.Tensor, values: torch.Tensor, sink: int, local: in
     tensors are its).  Returns the number of chunks.  Everything is bf16 and
     16-byte aligned (``cache_prefill_takes``)."""
     bs, kv, n, _ = keys.shape
-    n_max = chunk_min.shape[2]
+    n_rows, n_max, rs = k_rows.shape[2], chunk_min.shape[2], k_rows.stride()
     # the extents the kernel writes are k_rows' rows and chunk_min's chunks
     for name, t in (("k_rows", k_rows), ("v_rows", v_rows)):
-        _check_bf16(name, t)
-        if tuple(t.shape) != (bs, kv, k_rows.shape[2], HEAD_DIM) or t.stride(3) != 1 or t.stride(2) != HEAD_DIM \
-                or t.stride() != k_rows.stride():
+        if t.dtype != torch.bfloat16:
+            raise TypeError(f"{name} must be bfloat16; got {t.dtype}")
+        if t.shape != (bs, kv, n_rows, HEAD_DIM) or t.stride() != rs or rs[2:] != (HEAD_DIM, 1):
             raise ValueError(f"{name} must be [{bs}, {kv}, rows, {HEAD_DIM}] with contiguous rows, as k_rows; "
                              f"got {tuple(t.shape)} stride {t.stride()}")
-    for name, t, dtype, tail in (("chunk_min", chunk_min, torch.bfloat16, (HEAD_DIM,)),
-                                 ("chunk_max", chunk_max, torch.bfloat16, (HEAD_DIM,)),
-                                 ("chunk_centroid", chunk_centroid, torch.bfloat16, (HEAD_DIM,)),
-                                 ("chunk_valid", chunk_valid, torch.bool, ()),
-                                 ("packed_K", packed_K, torch.int32, (16, chunk_size))):
+    meta = (bs, kv, n_max, HEAD_DIM)
+    for name, t, dtype, shape in (("chunk_min", chunk_min, torch.bfloat16, meta),
+                                  ("chunk_max", chunk_max, torch.bfloat16, meta),
+                                  ("chunk_centroid", chunk_centroid, torch.bfloat16, meta),
+                                  ("chunk_valid", chunk_valid, torch.bool, meta[:3]),
+                                  ("packed_K", packed_K, torch.int32, meta[:3] + (16, chunk_size))):
         if t.dtype != dtype:
             raise TypeError(f"{name} must be {dtype}; got {t.dtype}")
-        if tuple(t.shape) != (bs, kv, n_max, *tail) or not t.is_contiguous():
-            raise ValueError(f"{name} must be contiguous {[bs, kv, n_max, *tail]}; got {tuple(t.shape)}")
+        if t.shape != shape or not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous {list(shape)}; got {tuple(t.shape)}")
     require_gpu(keys, values, k_rows, v_rows, chunk_min, chunk_max, chunk_centroid, chunk_valid, packed_K)
-    if any(t.device != keys.device for t in (k_rows, v_rows, chunk_min, chunk_max, chunk_centroid, chunk_valid, packed_K)):
-        raise ValueError("cache_prefill: all tensors on one device")
+    dev = keys.get_device()
+    for t in (k_rows, v_rows, chunk_min, chunk_max, chunk_centroid, chunk_valid, packed_K):
+        if t.get_device() != dev:
+            raise ValueError("cache_prefill: all tensors on one device")
     ret = n - sink - local
     if keys.shape != values.shape or ret < 0 or not cache_prefill_takes(keys, values):
         raise ValueError("cache_prefill: bf16 keys / values of one shape with 16-byte aligned rows")
-    ks, vs, rs = keys.stride(), values.stride(), k_rows.stride()
+    ks, vs = keys.stride(), values.stride()
     check(lib().zkv_cache_prefill(
         ptr(keys), ks[0], ks[1], ks[2], ptr(values), vs[0], vs[1], vs[2], bs, kv, sink, ret, local,
-        ptr(k_rows), ptr(v_rows), rs[0], rs[1], k_rows.shape[2], sink_row, ret_row, local_row, chunk_size, n_max,
+        ptr(k_rows), ptr(v_rows), rs[0], rs[1], n_rows, sink_row, ret_row, local_row, chunk_size, n_max,
         ptr(chunk_min), ptr(chunk_max), ptr(chunk_centroid), ptr(chunk_valid), ptr(packed_K), stream_of(keys)))
     return ret // chunk_size
 
 
 def cache_prefill_takes(*rows: torch.Tensor) -> bool:
     """Whether ``cache_prefill`` reads these [bs, kv, n, 128] tensors in place."""
-    return all(t.dtype == torch.bfloat16 and t.is_cuda and t.device == rows[0].device
-               and t.shape[-1] == HEAD_DIM and t.stride(-1) == 1 and not any(s % 8 for s in t.stride()[:3])
-               and t.data_ptr() % 16 == 0 and t.shape[2] < 2 ** 20
-               for t in rows)
+    dev = rows[0].device
+    for t in rows:
+        sb, sh, st, sd = t.stride()
+        if t.dtype != torch.bfloat16 or not t.is_cuda or t.device != dev or t.shape[3] != HEAD_DIM or sd != 1 \
+                or (sb | sh | st) & 7 or t.data_ptr() & 15 or t.shape[2] >= 2 ** 20:
+            return False
+    return True
 
 
 # ---------------------------------------------------------------------------
